@@ -855,24 +855,14 @@ __global__ __launch_bounds__(256) void attention_kv_f16_kernel(const float4v* k,
     }
 }
 
-// Split the key ranges only when the query tiles alone leave CUs idle, in the
-// shortest chunks whose work units still fit one round of workgroups (the
-// merge pass reads every unit's partial O back). At most 64 chunks per query
-// tile (the merge keeps their weights in LDS).
-void attention_plan(AttnParams& p, uint32_t cus)
+// The flash kernel's key split: units per head and the chunk length (units 0:
+// no split). Only when the query tiles alone leave CUs idle, in the shortest
+// chunks whose work units still fit one round of workgroups (the merge pass
+// reads every unit's partial O back). At most 64 chunks per query tile (the
+// merge keeps their weights in LDS).
+static void flash_split(AttnParams& p, uint32_t cus)
 {
     p.units = 0;
-    p.chunk_tiles = 0;
-    const uint32_t HD = p.head_dim;
-    const uint32_t qsz = p.q_dtype == DT_F32 ? 4 : 2;
-    // The flash kernel's operand rules (the reference's FA gate, attention.h:
-    // 916-945: Dh % 8 == 0, 16 <= Dh <= 256), plus 16-byte aligned operands
-    // and buffer ranges under 2^31 bytes; anything else takes the plain path.
-    const bool flash = HD % 8 == 0 && HD >= 16 && HD <= 256 && ((uintptr_t)p.q % 16) == 0 &&
-                       ((uintptr_t)p.k % 16) == 0 && ((uintptr_t)p.v % 16) == 0 &&
-                       (size_t)p.kv_rows * HD * 2 < (1ull << 31) && (size_t)p.tq * HD * qsz < (1ull << 31);
-    p.dp = !flash ? 0 : HD <= 64 ? 64 : HD <= 128 ? 128 : 256;
-    if (!p.dp) return;
     const uint32_t nqt = (p.tq + fa::BQ - 1) / fa::BQ, tiles = p.batch * p.hq * nqt;
     const uint32_t key_tiles = (plan_cached(p) + p.tkv + fa::BKV - 1) / fa::BKV;
     const uint32_t min_chunk = std::max<uint32_t>(2, (key_tiles + 63) / 64);
@@ -885,27 +875,31 @@ void attention_plan(AttnParams& p, uint32_t cus)
         if (wgs <= cus && wgs <= AttnParams::FA_WG_TAB && nqt <= 0x10000) {
             p.chunk_tiles = c;
             p.units = u;
-            // the units of a head, from the last query tile (the longest
-            // causal walks start first), chunk by chunk
-            uint32_t uq[AttnParams::FA_WG_TAB], uc[AttnParams::FA_WG_TAB], un[AttnParams::FA_WG_TAB], n = 0;
-            for (uint32_t qt = nqt; qt-- > 0;) {
-                const uint32_t nc = fa_chunks(p, qt, plan_cached(p));
-                p.qt_tab[qt] = n | nc << 16;
-                for (uint32_t ch = 0; ch < nc; ++ch, ++n) {
-                    uq[n] = qt;
-                    uc[n] = ch;
-                    un[n] = nc;
-                }
-            }
-            // workgroup w -> unit of head and batch, a head's units on one XCD
-            for (uint32_t w = 0; w < wgs; ++w) {
-                const uint32_t lb = fa_xcd_block(w, (uint32_t)wgs), unit = lb % u, h = (lb / u) % p.hq,
-                               b = lb / (u * p.hq);
-                p.wg_tab[2 * w] = uq[unit] | uc[unit] << 16 | un[unit] << 24;
-                p.wg_tab[2 * w + 1] = unit | h << 10 | b << 20;
-            }
             return;
         }
+    }
+}
+
+// The split launch's tables: the units of a head, from the last query tile
+// (the longest causal walks start first), chunk by chunk; workgroup w -> unit
+// of head and batch, a head's units on one XCD.
+static void flash_tables(AttnParams& p)
+{
+    const uint32_t nqt = (p.tq + fa::BQ - 1) / fa::BQ, u = p.units, wgs = u * p.batch * p.hq;
+    uint32_t uq[AttnParams::FA_WG_TAB], uc[AttnParams::FA_WG_TAB], un[AttnParams::FA_WG_TAB], n = 0;
+    for (uint32_t qt = nqt; qt-- > 0;) {
+        const uint32_t nc = fa_chunks(p, qt, plan_cached(p));
+        p.qt_tab[qt] = n | nc << 16;
+        for (uint32_t ch = 0; ch < nc; ++ch, ++n) {
+            uq[n] = qt;
+            uc[n] = ch;
+            un[n] = nc;
+        }
+    }
+    for (uint32_t w = 0; w < wgs; ++w) {
+        const uint32_t lb = fa_xcd_block(w, wgs), unit = lb % u, h = (lb / u) % p.hq, b = lb / (u * p.hq);
+        p.wg_tab[2 * w] = uq[unit] | uc[unit] << 16 | un[unit] << 24;
+        p.wg_tab[2 * w + 1] = unit | h << 10 | b << 20;
     }
 }
 
@@ -916,16 +910,42 @@ static size_t attention_kv_bytes(const AttnParams& p)
     return (2 * n * sizeof(half_t) + 255) & ~(size_t)255;
 }
 
+static size_t flash_workspace(const AttnParams& p)
+{
+    return attention_kv_bytes(p) +
+           (p.units ? (size_t)p.batch * p.hq * p.units * fa::BQ * (p.dp + 2) * sizeof(float) : 0);
+}
+
+// The path and its split: the plain kernel (dp 0), the decode kernel
+// (dec_units > 0) or the flash kernel.
+void attention_plan(AttnParams& p, uint32_t cus)
+{
+    p.units = 0;
+    p.chunk_tiles = 0;
+    p.dec_units = 0;
+    const uint32_t HD = p.head_dim;
+    const uint32_t qsz = p.q_dtype == DT_F32 ? 4 : 2;
+    // The flash kernel's operand rules (the reference's FA gate, attention.h:
+    // 916-945: Dh % 8 == 0, 16 <= Dh <= 256), plus 16-byte aligned operands
+    // and buffer ranges under 2^31 bytes; anything else takes the plain path.
+    const bool flash = HD % 8 == 0 && HD >= 16 && HD <= 256 && ((uintptr_t)p.q % 16) == 0 &&
+                       ((uintptr_t)p.k % 16) == 0 && ((uintptr_t)p.v % 16) == 0 &&
+                       (size_t)p.kv_rows * HD * 2 < (1ull << 31) && (size_t)p.tq * HD * qsz < (1ull << 31);
+    p.dp = !flash ? 0 : HD <= 64 ? 64 : HD <= 128 ? 128 : 256;
+    if (!p.dp) return;
+    flash_split(p, cus);
+    attention_decode_plan(p, cus, plan_cached(p) + p.tkv, flash_workspace(p));
+    if (p.dec_units == 0 && p.units) flash_tables(p);
+}
+
 size_t attention_workspace_bytes(const AttnParams& p)
 {
-    size_t bytes = attention_kv_bytes(p);
-    if (p.units) bytes += (size_t)p.batch * p.hq * p.units * fa::BQ * (p.dp + 2) * sizeof(float);
-    return bytes;
+    return p.dec_units ? attention_decode_workspace(p, p.dec_units) : flash_workspace(p);
 }
 
 void attention_set_workspace(AttnParams& p, void* ws)
 {
-    const size_t kvb = attention_kv_bytes(p);
+    const size_t kvb = p.dec_units ? 0 : attention_kv_bytes(p);
     p.ws_kv = kvb ? ws : nullptr;
     p.ws_o = (float*)((char*)ws + kvb);
     p.ws_ml = p.ws_o + (size_t)p.batch * p.hq * p.units * fa::BQ * p.dp;
@@ -958,7 +978,7 @@ static hipError_t attention_launch_d(const AttnParams& p, hipStream_t s)
 
 hipError_t attention_launch(const AttnParams& p0, hipStream_t s)
 {
-    if (p0.cache_count && p0.tkv > 0) {
+    if (p0.cache_count && p0.tkv > 0 && !(p0.dec_units && p0.dec_append)) {
         const size_t n = (size_t)p0.tkv * p0.head_dim;
         const uint32_t blocks = (uint32_t)std::min<size_t>((n + 255) / 256, 1024);
         hipLaunchKernelGGL(attention_append_kernel, dim3(blocks, p0.hkv), dim3(256), 0, s, p0);
@@ -969,6 +989,7 @@ hipError_t attention_launch(const AttnParams& p0, hipStream_t s)
         hipLaunchKernelGGL(attention_naive_kernel, dim3(p0.tq, p0.hq, p0.batch), dim3(256), 0, s, p0);
         return hipGetLastError();
     }
+    if (p0.dec_units) return attention_decode_launch(p0, s);
     AttnParams p = p0;
     if (p.kv_dtype == DT_F32) {
         if (!p.ws_kv) return hipErrorInvalidValue;

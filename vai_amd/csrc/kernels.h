@@ -201,7 +201,35 @@ struct AttnParams {
     // unit | its chunk count << 16 (a head has at most FA_WG_TAB units, so at
     // most that many query tiles)
     uint32_t qt_tab[FA_WG_TAB];
+    // Few query rows per KV head (attention_decode.hip): dec_units > 0 takes
+    // that path, with dec_rows = tq * hq / hkv rows per KV head, dec_rpb of
+    // them per workgroup; dec_append: it also appends the new rows.
+    uint32_t dec_units, dec_rows, dec_rpb, dec_append;
 };
+
+// The launch arguments of attention_decode.hip, from an AttnParams.
+struct AttnDecodeParams {
+    static constexpr uint32_t MAX_UNITS = 256;
+    void* out;
+    const void* q;
+    const void* k;
+    const void* v;
+    const void* k_new;            // the call's new rows [hkv, n_new, head_dim], attended and appended here
+    const void* v_new;
+    const uint32_t* cache_count;
+    float* ws_o;                  // [batch * hkv][units][rows][dp]
+    float* ws_ml;                 // [batch * hkv][units][rows][2]
+    int o_dtype, q_dtype, new_dtype;
+    uint32_t hq, hkv, tq, tkv, head_dim, kv_rows, ring;
+    uint32_t n_new;               // 0: no new rows, or appended before the launch
+    uint32_t rows, rpb, units;    // query rows per KV head, rows per workgroup, key chunks
+    float scale;
+    MaskRule mask;
+};
+void attention_decode_plan(AttnParams& p, uint32_t cus, uint32_t key_rows, size_t flash_workspace);
+size_t attention_decode_workspace(const AttnParams& p, uint32_t units);
+hipError_t attention_decode_launch(const AttnParams& p, hipStream_t s);
+
 bool attention_ok(const AttnParams& p);
 // Units per head for p's shape (0 when no query tile needs splitting), and
 // the workspace the split needs.
