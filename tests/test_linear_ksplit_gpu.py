@@ -1,0 +1,88 @@
+"""The small-tile Linear (gemm_ksplit.hip) against float64, at the edges of its
+tiles, k chunks and both staging forms. The bound is the rounding an fp32 sum
+of K exact products can make, K 2^-24 sum |x w|, plus one fp16 rounding of each
+fp32 activation (2^-11 sum |x w|) and of the output (2^-11 |y|)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from helpers import draw, normal
+
+pytestmark = pytest.mark.gpu
+F16, F32 = np.float16, np.float32
+
+
+def silu(v):
+    return v / (1 + np.exp(-v))
+
+
+def check(gpu, m, k, n, xdt, odt, tile, bias=None, residual=None, gated=False, off=0):
+    rng = np.random.default_rng(m + k + n)
+    w, x = draw(normal((n, k), 0.05), rng, F16), draw((m, k), rng, xdt)
+    b = draw(normal((n,) if bias == "row" else (m, n), 0.05), rng, F16) if bias else None
+    r = draw((n,) if residual == "row" else (m, n), rng, odt) if residual else None
+    D = gpu.DeviceArray.from_numpy
+    dw = D(np.concatenate([np.zeros(off, F16), w.ravel()]))
+    dx, db, dr = D(x), None if b is None else D(b), None if r is None else D(r)
+    out = gpu.DeviceArray((m, n // 2 if gated else n), odt)
+    out.fill_(0xFF)
+    a = gpu.linear_args(out, dx, D(w), db, dr, gated=gated, gate_epi="SILU")
+    a.weight = dw.ptr + 2 * off
+    name, splits = gpu.linear_plan(a)
+    print(f"ksplit m={m} k={k} n={n} {np.dtype(xdt)} -> {np.dtype(odt)} gated={gated} plan={name}", flush=True)
+    assert name == f"tile_f16_{tile}_kwaves" + ("_gated" if gated else "") and splits == 1
+    assert gpu.lib().vai_linear_workspace_size(ctypes.byref(a)) == 0
+    gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
+    gpu.synchronize()
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    mag = np.abs(x64) @ np.abs(w64).T
+    tol = mag * (k * 2.0 ** -24 + (2.0 ** -11 if xdt == F32 else 0)) + 1e-6
+    y = x64 @ w64.T + (0 if b is None else b.astype(np.float64))
+    if gated:
+        h = n // 2
+        g, u = y[:, :h], y[:, h:]
+        y = silu(g) * u
+        tol = 1.1 * tol[:, :h] * np.abs(u) + np.abs(silu(g)) * tol[:, h:] + 2e-6 * np.abs(y)   # |silu'| <= 1.1
+    elif r is not None:
+        y = y + r.astype(np.float64)
+    if odt == F16:
+        tol = tol + 2.0 ** -11 * np.abs(y)
+    got = out.numpy().astype(np.float64)
+    assert np.isfinite(got).all() and (np.abs(got - y) <= tol).all(), float((np.abs(got - y) / tol).max())
+
+
+@pytest.mark.parametrize("m, k, n, xdt, odt, tile, kw", [
+    (9, 32, 33, F16, F32, "32x32", {}),                             # one chunk, half of it past K; one column in the second tile
+    (32, 4096, 128, F16, F32, "32x32", {"bias": "row"}),            # every wave of eight runs whole trips
+    (33, 1032, 100, F16, F16, "32x32", {"residual": "full"}),       # a k tail of one 16-byte piece, a second row tile of one row
+    (50, 1000, 77, F32, F32, "32x32", {"bias": "row"}),             # fp32 X, odd N
+    (61, 1147, 96, F16, F32, "32x32", {"residual": "row"}),         # odd K: staged through registers
+    (70, 333, 40, F32, F16, "32x32", {"bias": "full"}),             # odd K, fp32 X, a bias of its own repeat
+    (64, 2048, 8192, F16, F16, "32x64", {"bias": "row", "residual": "full"}),
+    (90, 2040, 7000, F32, F32, "64x64", {}),
+    (61, 1148, 8191, F16, F32, "32x64", {"residual": "full"}),      # K % 8 = 4, odd N
+    (100, 1024, 5000, F16, F32, "64x64", {"residual": "full"}),
+    (300, 512, 4100, F16, F16, "64x128", {"bias": "row"}),          # quadrant tiles, ragged M and N
+    (300, 515, 4100, F32, F32, "64x128", {"residual": "full"}),     # ... through registers
+    (400, 576, 8192, F16, F32, "128x128", {"bias": "row"}),
+    (400, 571, 8192, F16, F16, "128x128", {}),
+    (511, 640, 8200, F32, F32, "128x128", {"residual": "full"}),
+])
+def test_ksplit(gpu, m, k, n, xdt, odt, tile, kw):
+    check(gpu, m, k, n, xdt, odt, tile, **kw)
+
+
+@pytest.mark.parametrize("m, k, h, xdt, odt, tile", [
+    (9, 256, 17, F16, F32, "32x32"),          # H one past a tile's 16 outputs
+    (40, 1000, 2050, F32, F16, "32x64"),
+    (61, 1021, 700, F16, F32, "32x32"),       # odd K
+    (300, 512, 2100, F16, F16, "64x128"),
+])
+def test_ksplit_gated(gpu, m, k, h, xdt, odt, tile):
+    check(gpu, m, k, 2 * h, xdt, odt, tile, bias="row", gated=True)
+
+
+def test_ksplit_unaligned_weight(gpu):
+    """A weight two bytes off a 16-byte boundary is staged through registers."""
+    check(gpu, 20, 512, 64, F16, F32, "32x32", off=1)

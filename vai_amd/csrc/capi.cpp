@@ -5,9 +5,10 @@
 // /root/reference/vai/nodes/linear.h:2101-2119; selectConvPlan,
 // /root/reference/vai/nodes/convolution.h:5408-5443) with one rule set for
 // gfx950: M <= 8 streams W through the slab GEMV (linear.h:320), larger M
-// takes the MFMA GEMM with the largest tile that still gives the 256 CUs at
-// least one workgroup each, and split-K when even the smallest tile leaves
-// most CUs idle and K is long.
+// takes an MFMA GEMM: 256x256 tiles for long prompts, the small-tile kernel
+// (gemm_ksplit.hip) below and for what those do not take, the fp32 kernel for
+// small fp32 problems, and the generic tiles for the rest (an fp32 weight, a
+// forced split).
 #include <cmath>
 #include <hip/hip_runtime.h>
 #include <stdio.h>
@@ -34,7 +35,8 @@ size_t dtype_bytes(int32_t d) { return d == VAI_DTYPE_F16 ? 2 : 4; }
 vai_status hip_status(hipError_t e) { return e == hipSuccess ? VAI_OK : (vai_status)e; }
 
 struct LinearPlan {
-    enum Kind { Slab, SlabThenGate, Tile, BigTile, PackedTile, F32Small, Acc16Tile } kind;
+    enum Kind { Slab, SlabThenGate, Tile, BigTile, PackedTile, F32Small, Acc16Tile, KSplit } kind;
+    int ks_tile;        // KSplit: which tile
     bool packed_gemv;   // Slab / SlabThenGate over the packed weight
     GemmTile tile;
     uint32_t bm, bn;
@@ -109,6 +111,17 @@ uint32_t acc16_guess_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t cores)
 
 namespace {
 
+// The packed 256x256 kernel's time (us) on g: rounds of units, 1.77 us per
+// 64-wide k stage (config 3: 512 tiles, 48 stages, 177 us), and with a K split
+// the reduce launch and its passes over the partial planes (M = 2000,
+// K = N = 2048 in 4 splits: 43 us, of which the planes are 20).
+float packed_us(const GemmParams& g, bool gated, uint32_t tiles)
+{
+    const uint32_t S = gated ? 1 : g.splits, rounds = (tiles * S + plan_cus() - 1) / plan_cus();
+    const float us = 2.5f + rounds * (4.f + 1.77f * (float)(g.K / S) / 64.f);
+    return S == 1 ? us : us + 4.f + (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 4e6f;
+}
+
 LinearPlan plan_linear(const vai_linear_args* a)
 {
     LinearPlan p{};
@@ -145,6 +158,14 @@ LinearPlan plan_linear(const vai_linear_args* a)
         GemmParams g{};
         g.a_dtype = a->i_dtype; g.b_dtype = a->w_dtype; g.M = M; g.N = N; g.K = K; g.H = a->gated ? N / 2 : 0;
         g.A = a->in; g.B = a->weight; g.splits = 1; g.batch = 1;
+        // The small-tile kernel with its best tile and modelled time: for
+        // whatever the 256x256 kernels do not take, and where it is faster
+        // than the packed one below 512 rows or when that would need more than
+        // 8 K splits (their planes then cost more than the product: M = 608,
+        // K = 3072, N = 896 in 12 splits 124 us against 19).
+        float ksplit_us = 0.f;
+        const bool ksplit = a->split_size == 0 && gemm_ksplit_ok(g, a->gated != 0);
+        if (ksplit) p.ks_tile = gemm_ksplit_plan(g, a->gated != 0, plan_cus(), &ksplit_us);
         if (a->split_size == 0 && a->packed_weight) {
             // Fewer 256x256 tiles than half the CUs (a down projection: M=2048,
             // N=3072 is 96 tiles): split K so the units fill the chip, the
@@ -156,7 +177,8 @@ LinearPlan plan_linear(const vai_linear_args* a)
                 while (splits > 1 && K % (splits * 128) != 0) --splits;
             }
             g.splits = splits;
-            if (gemm_packed_ok(g, a->gated)) {
+            const bool small = M < 512 || splits > 8;
+            if (gemm_packed_ok(g, a->gated) && !(small && ksplit && ksplit_us < packed_us(g, a->gated != 0, tiles))) {
                 p.kind = LinearPlan::PackedTile;
                 p.splits = splits;
                 p.split_size = K / splits;
@@ -172,6 +194,13 @@ LinearPlan plan_linear(const vai_linear_args* a)
             p.kind = LinearPlan::F32Small;
             p.bm = 32;
             p.bn = 16 * nf;
+            p.splits = 1;
+            p.split_size = K;
+            p.workspace = 0;
+            return p;
+        }
+        if (ksplit && !(M >= 512 && gemm_big_ok(g, a->gated))) {
+            p.kind = LinearPlan::KSplit;
             p.splits = 1;
             p.split_size = K;
             p.workspace = 0;
@@ -269,6 +298,10 @@ vai_status vai_linear_plan(const vai_linear_args* a, char* name, size_t name_len
     } else if (p.kind == LinearPlan::BigTile || p.kind == LinearPlan::PackedTile) {
         snprintf(buf, sizeof buf, "tile_f16_256x256%s%s", p.kind == LinearPlan::PackedTile ? "_packed" : "",
                  a->gated ? "_gated" : "");
+    } else if (p.kind == LinearPlan::KSplit) {
+        uint32_t bm, bn;
+        gemm_ksplit_tile(p.ks_tile, bm, bn);
+        snprintf(buf, sizeof buf, "tile_f16_%ux%u_kwaves%s", bm, bn, a->gated ? "_gated" : "");
     } else {
         const bool f32 = a->i_dtype == VAI_DTYPE_F32 && a->w_dtype == VAI_DTYPE_F32;
         snprintf(buf, sizeof buf, "tile_%s_%s%s", f32 ? "f32" : "f16", tile_name(p.tile, a->gated),
@@ -338,7 +371,7 @@ static vai_status linear_run(const vai_linear_args* a, const LinearPlan& p, hipS
                                                a->gate_epilogue, a->N, s));
     }
     if (p.kind == LinearPlan::F32Small) return hip_status(gemm_f32_launch(g, (int)(p.bn / 16), s));
-    hipError_t e = gemm_launch(g, a->gated ? BKind::Gated : BKind::Dense,
+    hipError_t e = p.kind == LinearPlan::KSplit ? gemm_ksplit_launch(g, a->gated != 0, p.ks_tile, s) : gemm_launch(g, a->gated ? BKind::Gated : BKind::Dense,
                                a->gated ? EpiKind::Gated : EpiKind::Linear, p.tile, s);
     if (e != hipSuccess || p.splits == 1) return hip_status(e);
     const size_t MN = (size_t)a->M * (a->gated ? a->N / 2 : a->N);

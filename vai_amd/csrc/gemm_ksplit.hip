@@ -1,0 +1,635 @@
+// gemm_ksplit.hip -- the fp16 MFMA Linear for every size between the GEMV and
+// the 256x256 tiles: X (fp16 or fp32) . W^T (fp16, as stored), any N and K,
+// fused gate/up included.
+//
+// What bounds these sizes is bytes into the CUs (W and X each pass through
+// LDS once per workgroup, about 45 bytes a cycle and CU) and how many CUs have
+// work, not MFMA rate. So the output is cut into small tiles (32x32 to
+// 128x128, chosen by gemm_ksplit_plan so that the tiles fill the CUs), and the
+// 4 or 8 waves of a workgroup split K instead of the tile: every wave runs the
+// whole tile over its own 64- or 32-wide k chunks, dealt out in turn, so each
+// staged byte is written to LDS once and read from it once (a 2x2 split of the
+// tile reads each operand twice), no wave waits for another in the K loop,
+// and small tiles still keep four to eight waves' copies in flight. Each wave
+// has its own ring of stages filled by buffer_load ... lds (whole 64- to
+// 256-byte row pieces, 16-byte chunks XOR-swizzled by row); the partial tiles
+// meet in LDS at the end. fp32 X is copied as fp32 and rounded to fp16 when
+// its fragments are read (once, since no two waves read the same k), the
+// rounding the tile path's fp16 staging always made.
+//
+// Tiles of 64x128 up are quadrants of four waves over one shared ring instead:
+// their partial tiles would not fit LDS, and 64 k of both operands a wave only
+// once each. The copies are spread over the MFMA steps (in one burst a stage
+// took 0.56 us at 128x128, spread 0.40).
+//
+// Measured (back-to-back calls, us, against the kernels these sizes took
+// before, register-staged 64x64 tiles or 256x256 packed tiles with a K split):
+// X fp16 [61, 3072], N 5120 20.2 -> 11.1 (2.9 TB/s of W); fp32 [500, 2048],
+// N 2048 65.2 -> 15.0; fp16 [300, 4096], N 1000 146 -> 12; fp16 [948, 2481],
+// N 1216 (odd K) 205 -> 28; gated fp16 [500, 2048], H 2048 71 -> 16. At 32x32
+// a workgroup moves 8.7 us per MB of its operands, 50 bytes a cycle.
+//
+// Rows that are not whole 16-byte chunks (K % 8 != 0) or operands off a
+// 16-byte boundary take the same kernel with the chunks loaded into registers
+// (unaligned 16-byte loads, the last chunk of a row element by element) and
+// written to LDS from there.
+#include <algorithm>
+
+#include "device_common.h"
+#include "kernels.h"
+#include "launch_once.h"
+
+#define LDS_AS __attribute__((address_space(3)))
+
+namespace vai_dev {
+
+namespace ks {
+
+// One variant: tile, waves, k per stage and ring depth for X of type TA.
+// KSP: the waves split K, each with its own ring; otherwise four waves take a
+// quadrant each of the tile and share one ring. DMA false: staged through
+// registers (one stage per wave, or two shared ones), X in LDS as fp16.
+template <int BM_, int BN_, int NW_, int BK_, int S_, bool KSP_, typename TA_, bool DMA_>
+struct Cfg {
+    static constexpr int BM = BM_, BN = BN_, NW = NW_, BK = BK_, S = DMA_ ? S_ : (KSP_ ? 1 : 2);
+    static constexpr bool KSP = KSP_, DMA = DMA_;
+    typedef TA_ TA;
+    static constexpr int WM = KSP ? BM : BM / 2, WN = KSP ? BN : BN / 2;   // a wave's part of the tile
+    // sums per output and wave (k steps in turn)
+    static constexpr int AS = !KSP ? 1 : WM * WN <= 32 * 64 ? (BK / 16 < 4 || NW == 8 ? 2 : 4) : 2;
+    static constexpr int AES = DMA ? (int)sizeof(TA) : 2;      // X element bytes in LDS
+    static constexpr int AROW = BK * AES, BROW = BK * 2;       // row bytes in LDS
+    static constexpr int ABYTES = BM * AROW, BBYTES = BN * BROW, STAGE = ABYTES + BBYTES;
+    static constexpr int SHARE = KSP ? 1 : NW;                 // waves that fill a stage together
+    static constexpr int ACOPIES = ABYTES / 1024 / SHARE, BCOPIES = BBYTES / 1024 / SHARE, COPIES = ACOPIES + BCOPIES;
+    static constexpr int RING = (KSP ? NW : 1) * S * STAGE;
+    // the final exchange: RB rows of every partial tile at a time
+    static constexpr int PLANES = KSP ? NW : 1;
+    static constexpr int RROW = BN * 4 + 16;
+    static constexpr int RB = PLANES * BM * RROW <= 160 * 1024 ? BM : BM / 2;
+    static constexpr int RED = PLANES * RB * RROW;
+    static constexpr int LDS = RING > RED ? RING : RED;
+    static_assert(LDS <= 160 * 1024 && RB % 32 == 0 && ACOPIES * SHARE * 1024 == ABYTES &&
+                  BCOPIES * SHARE * 1024 == BBYTES && (KSP || (NW == 4 && RB == BM)), "fits");
+};
+
+// Physical 16-byte chunk of logical chunk c in row r, rows of ROWB bytes: the
+// 16 rows one pass of a 16-byte fragment read touches land on 16 distinct
+// chunks of the 256-byte bank window.
+template <int ROWB>
+__device__ __forceinline__ int swz(int r, int c)
+{
+    constexpr int CH = ROWB / 16, RPW = ROWB >= 256 ? 1 : 256 / ROWB;
+    return c ^ ((r / RPW) % CH);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+__device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14)); }
+
+// 8 elements at any alignment, as fp16
+template <typename T>
+__device__ __forceinline__ half8 load8(const T* p)
+{
+    if constexpr (sizeof(T) == 2) {
+        typedef half8 half8u __attribute__((aligned(2)));
+        return *(const half8u*)p;
+    } else {
+        typedef float4v float4u __attribute__((aligned(4)));
+        const float4v lo = *(const float4u*)p, hi = *(const float4u*)(p + 4);
+        return __builtin_shufflevector(__builtin_convertvector(lo, half4), __builtin_convertvector(hi, half4), 0, 1, 2,
+                                       3, 4, 5, 6, 7);
+    }
+}
+
+// v moved down by s elements (0 .. 8), zeros from above
+__device__ __forceinline__ half8 shift_down(half8 v, uint32_t s)
+{
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 w = __builtin_bit_cast(u32x4, v);
+    const uint32_t d = s >> 1;
+    uint32_t x[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        x[i] = 0;
+#pragma unroll
+        for (int k = 0; k + i < 4; ++k) x[i] = d == (uint32_t)k ? w[i + k] : x[i];
+    }
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (s & 1) ? (x[i] >> 16) | (x[i + 1] << 16) : x[i];
+    return __builtin_bit_cast(half8, r);
+}
+
+}   // namespace ks
+
+template <typename C, bool GATED>
+__global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_kernel(GemmParams p)
+{
+    using namespace ks;
+    constexpr int BM = C::BM, BN = C::BN, NW = C::NW, BK = C::BK, S = C::S;
+    constexpr int FM = C::WM / 32, FN = C::WN / 32, KSTEPS = BK / 16;
+    constexpr int BNO = GATED ? BN / 2 : BN;    // output columns per tile
+    constexpr int TH = 64 * NW;
+    typedef typename C::TA TA;
+    extern __shared__ half8 ks_lds[];
+    LDS_AS char* lds = (LDS_AS char*)(LDS_AS void*)ks_lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 31, fk = lane >> 5;
+    const uint32_t M = p.M, N = p.N, K = p.K, H = p.H, NO = GATED ? H : N;
+    const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = (NO + BNO - 1) / BNO, tiles = tiles_m * tiles_n;
+
+    // Workgroup -> tile. Workgroups go round-robin over the 8 XCDs; each XCD
+    // takes a contiguous run of the tiles, ordered so that the
+    // operand with more bytes is cut up among the XCDs and the other one is
+    // what every XCD's L2 reads whole.
+    const uint32_t w = blockIdx.x, x = w % 8, q8 = tiles / 8, r8 = tiles % 8;
+    const uint32_t t = x * q8 + (x < r8 ? x : r8) + w / 8;
+    const bool nmaj = (uint64_t)NO * (GATED ? 4 : 2) >= (uint64_t)M * sizeof(TA);
+    const uint32_t tm = __builtin_amdgcn_readfirstlane(nmaj ? t % tiles_m : t / tiles_n);
+    const uint32_t tn = __builtin_amdgcn_readfirstlane(nmaj ? t / tiles_m : t % tiles_n);
+    const uint32_t m0 = tm * BM, n0 = tn * BNO;
+    const int chunks = (int)((K + BK - 1) / BK);
+    // the chunks this wave runs: all, or wave, wave + NW, ..
+    const int mine = C::KSP ? (chunks - wave + NW - 1) / NW : chunks;
+    const int wm0 = C::KSP ? 0 : (wave >> 1) * C::WM, wn0 = C::KSP ? 0 : (wave & 1) * C::WN;
+
+    const TA* A = (const TA*)p.A;
+    const half_t* B = (const half_t*)p.B;
+    // W row of the tile's logical column j (clamped into W; a column past the
+    // output is never stored)
+    const auto wrow = [&](uint32_t j) __attribute__((always_inline)) {
+        if constexpr (GATED) {
+            const uint32_t c = n0 + (j < BNO ? j : j - BNO);
+            return std::min(c, H - 1) + (j < BNO ? 0u : H);
+        } else {
+            return std::min(n0 + j, N - 1);
+        }
+    };
+
+    LDS_AS char* ring = lds + (C::KSP ? wave * S * C::STAGE : 0);
+    const int cw = C::KSP ? 0 : wave;   // which share of a stage's copies is this wave's
+
+    // ---- staging ----
+    // Copy slot s of an operand (16 bytes) holds row s / CH, physical chunk
+    // s % CH. Rows past M read as zero (out of the resource's range), chunks
+    // past the row's end too (an offset past any range).
+    constexpr int ACH = C::AROW / 16, BCH = C::BROW / 16;
+    constexpr int AEC = 16 / C::AES;            // X elements per chunk
+    uint32_t aoff[C::ACOPIES], boff[C::BCOPIES];
+    __amdgpu_buffer_rsrc_t ra, rb;
+    half8 sa[C::DMA ? 1 : C::ACOPIES], sb[C::DMA ? 1 : C::BCOPIES];
+    if constexpr (C::DMA) {
+        ra = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(A + (size_t)m0 * K), (short)0,
+                                               (int)__builtin_amdgcn_readfirstlane((M - m0) * K * (uint32_t)sizeof(TA)),
+                                               0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)uniform_ptr(B), (short)0, (int)__builtin_amdgcn_readfirstlane((GATED ? 2 * H : N) * K * 2), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < C::ACOPIES; ++i) {
+            const int s = (cw * C::ACOPIES + i) * 64 + lane, row = s / ACH, ch = swz<C::AROW>(row, s % ACH);
+            aoff[i] = ((uint32_t)row * K + ch * AEC) * sizeof(TA);
+        }
+#pragma unroll
+        for (int i = 0; i < C::BCOPIES; ++i) {
+            const int s = (cw * C::BCOPIES + i) * 64 + lane, row = s / BCH, ch = swz<C::BROW>(row, s % BCH);
+            boff[i] = (wrow(row) * K + ch * 8) * 2;
+        }
+    }
+    // Part q of KSTEPS of this wave's copies of chunk c into a slot, spread over
+    // the MFMA steps (a burst holds the wave about 100 cycles a copy on the
+    // vector memory path). Chunks past the range copy zeros, so that the
+    // number of copies in flight stays fixed.
+    const auto issue_part = [&](int slot, int c, int q) __attribute__((always_inline)) {
+        const uint32_t k0 = (uint32_t)c * BK;
+        const uint32_t left = c < chunks ? K - k0 : 0u;
+        LDS_AS char* adst = ring + slot * C::STAGE + cw * C::ACOPIES * 1024;
+        LDS_AS char* bdst = ring + slot * C::STAGE + C::ABYTES + cw * C::BCOPIES * 1024;
+#pragma unroll
+        for (int i = C::ACOPIES * q / KSTEPS; i < C::ACOPIES * (q + 1) / KSTEPS; ++i) {
+            const int s = (cw * C::ACOPIES + i) * 64 + lane, ch = swz<C::AROW>(s / ACH, s % ACH);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_AS void*)(adst + i * 1024), 16,
+                                                     (int)((uint32_t)ch * AEC < left ? aoff[i] : 0x80000000u),
+                                                     (int)(k0 * sizeof(TA)), 0, 0);
+        }
+#pragma unroll
+        for (int i = C::BCOPIES * q / KSTEPS; i < C::BCOPIES * (q + 1) / KSTEPS; ++i) {
+            const int s = (cw * C::BCOPIES + i) * 64 + lane, ch = swz<C::BROW>(s / BCH, s % BCH);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_AS void*)(bdst + i * 1024), 16,
+                                                     (int)((uint32_t)ch * 8 < left ? boff[i] : 0x80000000u),
+                                                     (int)(k0 * 2), 0, 0);
+        }
+    };
+    const auto issue = [&](int slot, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < KSTEPS; ++q) issue_part(slot, c, q);
+    };
+    // Register staging of chunk c, and its write into a stage. Rows past M
+    // read row M - 1 (their outputs are never stored); a piece past the row's
+    // last 8 elements reads those and moves them down.
+    const auto fetch = [&](int c) __attribute__((always_inline)) {
+        const uint32_t k0 = (uint32_t)c * BK;
+        const bool whole = k0 + BK <= K;
+#pragma unroll
+        for (int i = 0; i < C::ACOPIES; ++i) {
+            const int s = (cw * C::ACOPIES + i) * 64 + lane;
+            const uint32_t k = k0 + (s % ACH) * 8, m = std::min(m0 + s / ACH, M - 1);
+            sa[i] = load8(A + (size_t)m * K + std::min(k, K - 8));
+        }
+#pragma unroll
+        for (int i = 0; i < C::BCOPIES; ++i) {
+            const int s = (cw * C::BCOPIES + i) * 64 + lane;
+            const uint32_t k = k0 + (s % BCH) * 8;
+            sb[i] = load8(B + (size_t)wrow(s / BCH) * K + std::min(k, K - 8));
+        }
+        if (!whole) {
+#pragma unroll
+            for (int i = 0; i < C::ACOPIES; ++i) {
+                const uint32_t k = k0 + (((cw * C::ACOPIES + i) * 64 + lane) % ACH) * 8;
+                sa[i] = shift_down(sa[i], std::min(k - std::min(k, K - 8), 8u));
+            }
+#pragma unroll
+            for (int i = 0; i < C::BCOPIES; ++i) {
+                const uint32_t k = k0 + (((cw * C::BCOPIES + i) * 64 + lane) % BCH) * 8;
+                sb[i] = shift_down(sb[i], std::min(k - std::min(k, K - 8), 8u));
+            }
+        }
+    };
+    const auto place = [&](int slot) __attribute__((always_inline)) {
+        LDS_AS char* st = ring + slot * C::STAGE;
+#pragma unroll
+        for (int i = 0; i < C::ACOPIES; ++i) {
+            const int s = (cw * C::ACOPIES + i) * 64 + lane, row = s / ACH;
+            *(LDS_AS half8*)(st + row * C::AROW + swz<C::AROW>(row, s % ACH) * 16) = sa[i];
+        }
+#pragma unroll
+        for (int i = 0; i < C::BCOPIES; ++i) {
+            const int s = (cw * C::BCOPIES + i) * 64 + lane, row = s / BCH;
+            *(LDS_AS half8*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, s % BCH) * 16) = sb[i];
+        }
+    };
+
+    // ---- fragments: row i*32 + fr of the wave's part, 16-wide k step q ----
+    const auto read_x = [&](const LDS_AS char* st, int i, int q) __attribute__((always_inline)) {
+        const int row = wm0 + i * 32 + fr;
+        if constexpr (C::AES == 2) {
+            return *(const LDS_AS half8*)(st + row * C::AROW + swz<C::AROW>(row, q * 2 + fk) * 16);
+        } else {
+            const float4v lo = *(const LDS_AS float4v*)(st + row * C::AROW + swz<C::AROW>(row, q * 4 + 2 * fk) * 16);
+            const float4v hi = *(const LDS_AS float4v*)(st + row * C::AROW + swz<C::AROW>(row, q * 4 + 2 * fk + 1) * 16);
+            return __builtin_shufflevector(__builtin_convertvector(lo, half4), __builtin_convertvector(hi, half4), 0, 1,
+                                           2, 3, 4, 5, 6, 7);
+        }
+    };
+    const auto read_w = [&](const LDS_AS char* st, int j, int q) __attribute__((always_inline)) {
+        const int row = wn0 + j * 32 + fr;
+        return *(const LDS_AS half8*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, q * 2 + fk) * 16);
+    };
+
+    // This thread's output columns in the final exchange (the same for each of
+    // its rows), and their bias, loaded ahead of the K loop.
+    constexpr int CG = BNO / 4;                 // 4-column groups per output row
+    const uint32_t cg = threadIdx.x % CG, col = n0 + 4 * cg;
+    const bool row_bias = !p.bias || p.bias_repeat == (GATED ? 2 * H : N);
+    float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias && row_bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t c = std::min(col + e, NO - 1);
+            bg[e] = ld(p.bias, p.bias_dtype, c);
+            if constexpr (GATED) bu[e] = ld(p.bias, p.bias_dtype, H + c);
+        }
+    }
+
+    // D = W X^T: lane (fr, fk) holds X row i*32 + fr at columns j*32 + 8 g + 4 fk .. +3.
+    // The k steps go to AS sums in turn: with the waves' own K shares at
+    // least 8 shorter chains per output, as exact as a split-K launch with
+    // its planes summed (K = 4096: 1.3e-7 relative; one chain a wave 1.6e-7).
+    constexpr int AS = C::AS;
+    float16v acc[AS][FM][FN];
+#pragma unroll
+    for (int a = 0; a < AS; ++a)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[a][i][j] = (float16v)0.f;
+
+    // A stage's MFMAs; step(q) runs after those of k step q. KSP reads all of
+    // the stage's fragments first (so that its slot can be refilled during the
+    // MFMAs), the shared ring's waves read one step ahead.
+    const auto stage_mfma = [&](const LDS_AS char* st, auto&& step) __attribute__((always_inline)) {
+        constexpr int AHEAD = C::KSP ? KSTEPS : 1, SETS = C::KSP ? KSTEPS : 2;
+        half8 xf[SETS][FM], wf[SETS][FN];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i) xf[q][i] = read_x(st, i, q);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) wf[q][j] = read_w(st, j, q);
+        }
+        if constexpr (C::KSP && C::DMA) wait_lgkmcnt0();
+#pragma unroll
+        for (int q = 0; q < KSTEPS; ++q) {
+            if (q + AHEAD < KSTEPS) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) xf[(q + AHEAD) % SETS][i] = read_x(st, i, q + AHEAD);
+#pragma unroll
+                for (int j = 0; j < FN; ++j) wf[(q + AHEAD) % SETS][j] = read_w(st, j, q + AHEAD);
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[q % AS][i][j] =
+                        __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[q % SETS][j], xf[q % SETS][i], acc[q % AS][i][j], 0, 0, 0);
+            if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
+            step(q);
+            if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    if constexpr (C::DMA && C::KSP) {
+        // Stage r of this wave is its chunk wave + r NW. S stages are in
+        // flight or being read: at the top of trip r stages r .. r + S - 1 are
+        // issued, so once at most (S - 1) COPIES copies are outstanding stage r
+        // has landed. Its slot is refilled when every read of it returned.
+#pragma unroll
+        for (int r = 0; r < S; ++r) issue(r, wave + r * NW);
+        int slot = 0;
+        for (int r = 0; r < mine; ++r) {
+            wait_vmcnt<(S - 1) * C::COPIES>();
+            stage_mfma(ring + slot * C::STAGE, [&](int q) __attribute__((always_inline)) {
+                issue_part(slot, wave + (r + S) * NW, q);
+            });
+            slot = slot + 1 == S ? 0 : slot + 1;
+        }
+        wait_vmcnt<0>();   // the copies past the range land before LDS is reused
+    } else if constexpr (C::DMA) {
+        // Stages r .. r + S - 2 are issued at the top of trip r: once at most
+        // (S - 2) COPIES of this wave's copies are outstanding its share of
+        // stage r has landed, after the barrier every wave's has, and every
+        // wave is done reading stage r - 1 (its reads returned before the
+        // barrier), whose slot takes stage r + S - 1.
+#pragma unroll
+        for (int r = 0; r < S - 1; ++r) issue(r, r);
+        int slot = 0;
+        for (int r = 0; r < mine; ++r) {
+            wait_vmcnt<(S - 2) * C::COPIES>();
+            wait_lgkmcnt0();
+            __builtin_amdgcn_s_barrier();
+            const int free = slot == 0 ? S - 1 : slot - 1;
+            stage_mfma(ring + slot * C::STAGE,
+                       [&](int q) __attribute__((always_inline)) { issue_part(free, r + S - 1, q); });
+            slot = slot + 1 == S ? 0 : slot + 1;
+        }
+        wait_vmcnt<0>();   // the copies past the range land before LDS is reused
+    } else if constexpr (C::KSP) {
+        if (mine > 0) fetch(wave);
+        for (int r = 0; r < mine; ++r) {
+            place(0);
+            if (r + 1 < mine) fetch(wave + (r + 1) * NW);
+            stage_mfma(ring, [](int) {});
+        }
+    } else {
+        // A wave that writes stage r + 2 has passed the barrier of trip
+        // r + 1, so every wave is done reading stage r from the same slot.
+        fetch(0);
+        for (int r = 0; r < mine; ++r) {
+            place(r & 1);
+            if (r + 1 < mine) fetch(r + 1);
+            __syncthreads();
+            stage_mfma(ring + (r & 1) * C::STAGE, [](int) {});
+        }
+    }
+
+#pragma unroll
+    for (int a = 1; a < AS; ++a)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[0][i][j] += acc[a][i][j];
+
+    // ---- the partial tiles meet in LDS, RB rows at a time ----
+    // U rows of a thread's four columns at a time, the residual of the next U
+    // loaded ahead; as vectors where rows are whole aligned groups of four
+    // (`al`). A bias or residual with its own repeat goes element by element.
+    const bool al = NO % 4 == 0 && ((uintptr_t)p.C % 16) == 0 && ((uintptr_t)p.residual % 16) == 0;
+    const bool batch = row_bias && (!p.residual || p.residual_repeat == 0);
+    const bool res = !GATED && p.residual;
+    constexpr int RSTEP = TH / CG, RT = C::RB > RSTEP ? C::RB / RSTEP : 1;   // rows per thread and round
+    constexpr int U = RT < 4 ? RT : 4;
+    static_assert(RT % U == 0, "whole groups of rows");
+    const uint32_t r0 = threadIdx.x / CG;
+#pragma unroll
+    for (int h = 0; h < BM / C::RB; ++h) {
+        float4v rv[U];
+        const auto residual = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const uint32_t row = std::min(m0 + h * C::RB + r0 + (t0 + i) * RSTEP, M - 1);
+                const size_t o = (size_t)row * NO + (al ? std::min(col, NO - 4) : 0u);
+                if (!al) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rv[i][e] = ld(p.residual, p.residual_dtype, o + std::min(col + e, NO - 1));
+                } else if (p.residual_dtype == DT_F16)
+                    rv[i] = __builtin_convertvector(*(const half4*)((const half_t*)p.residual + o), float4v);
+                else
+                    rv[i] = *(const float4v*)((const float*)p.residual + o);
+            }
+        };
+        if (batch && res) residual(0);
+        __syncthreads();
+#pragma unroll
+        for (int i = C::KSP ? h * (C::RB / 32) : 0; i < (C::KSP ? (h + 1) * (C::RB / 32) : FM); ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int row = (C::KSP ? wave * C::RB : wm0) + i * 32 + fr - h * C::RB;
+                    *(LDS_AS float4v*)(lds + row * C::RROW + (wn0 + j * 32 + 8 * g + 4 * fk) * 4) =
+                        float4v{acc[0][i][j][4 * g], acc[0][i][j][4 * g + 1], acc[0][i][j][4 * g + 2], acc[0][i][j][4 * g + 3]};
+                }
+        __syncthreads();
+        const auto sums = [&](uint32_t rr, float4v& v, float4v& up) __attribute__((always_inline)) {
+            v = up = (float4v)0.f;
+#pragma unroll
+            for (int w2 = 0; w2 < C::PLANES; ++w2) {
+                const LDS_AS char* src = lds + (w2 * C::RB + rr) * C::RROW + cg * 16;
+                v += *(const LDS_AS float4v*)src;
+                if constexpr (GATED) up += *(const LDS_AS float4v*)(src + BNO * 4);
+            }
+        };
+        if (batch) {
+#pragma unroll 1
+            for (int t0 = 0; t0 < RT; t0 += U) {
+                float4v v[U], up[U], rc[U];
+#pragma unroll
+                for (int i = 0; i < U; ++i) {
+                    sums(std::min<uint32_t>(r0 + (t0 + i) * RSTEP, C::RB - 1), v[i], up[i]);
+                    rc[i] = res ? rv[i] : (float4v)0.f;
+                }
+                if (res && t0 + U < RT) residual(t0 + U);
+                const auto rows = [&](auto&& put) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < U; ++i) {
+                        const uint32_t rr = r0 + (t0 + i) * RSTEP, row = m0 + h * C::RB + rr;
+                        if (rr < C::RB && row < M && col < NO) put(i, row);
+                    }
+                };
+                const auto act = [&](auto EPI) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < U; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if constexpr (GATED) v[i][e] = epilogue(v[i][e] + bg[e], EPI) * (up[i][e] + bu[e]);
+                            else v[i][e] = finish(v[i][e] + bg[e], rc[i][e], EPI, p.residual_order, p.scalar_scale);
+                        }
+                };
+                switch (p.epilogue) {
+                case 0: act(std::integral_constant<uint32_t, 0>{}); break;
+                case 1: act(std::integral_constant<uint32_t, 1>{}); break;
+                case 2: act(std::integral_constant<uint32_t, 2>{}); break;
+                case 3: act(std::integral_constant<uint32_t, 3>{}); break;
+                case 4: act(std::integral_constant<uint32_t, 4>{}); break;
+                default: act(std::integral_constant<uint32_t, 5>{}); break;
+                }
+                if (!al)
+                    rows([&](int i, uint32_t row) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (col + e < NO) st(p.C, p.c_dtype, (size_t)row * NO + col + e, v[i][e]);
+                    });
+                else if (p.c_dtype == DT_F16)
+                    rows([&](int i, uint32_t row) __attribute__((always_inline)) {
+                        *(half4*)((half_t*)p.C + (size_t)row * NO + col) = __builtin_convertvector(v[i], half4);
+                    });
+                else
+                    rows([&](int i, uint32_t row) __attribute__((always_inline)) {
+                        *(float4v*)((float*)p.C + (size_t)row * NO + col) = v[i];
+                    });
+            }
+        } else {
+#pragma unroll 1
+            for (uint32_t rr = r0; rr < C::RB; rr += RSTEP) {
+                const uint32_t row = m0 + h * C::RB + rr;
+                if (row >= M) break;
+                float4v v, up;
+                sums(rr, v, up);
+#pragma unroll 1
+                for (uint32_t e = 0; e < 4 && col + e < NO; ++e) {
+                    const float x = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
+                    const float y = e == 0 ? up[0] : e == 1 ? up[1] : e == 2 ? up[2] : up[3];
+                    const uint32_t c = col + e;
+                    const size_t o = (size_t)row * NO + c;
+                    if constexpr (GATED) {
+                        const float g0 = p.bias ? ld(p.bias, p.bias_dtype, c) : 0.f;
+                        const float u0 = p.bias ? ld(p.bias, p.bias_dtype, H + c) : 0.f;
+                        st(p.C, p.c_dtype, o, epilogue(x + g0, p.epilogue) * (y + u0));
+                    } else {
+                        store_output_general(OutputSpec{p.C, p.bias, p.residual, p.c_dtype, p.bias_dtype, p.bias_repeat,
+                                                        p.residual_repeat, p.epilogue, p.residual_order, p.scalar_scale},
+                                             o, x);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// fp16 W, fp16 or fp32 X, 32-bit buffer offsets.
+bool gemm_ksplit_ok(const GemmParams& p, bool gated)
+{
+    const uint64_t as = p.a_dtype == DT_F16 ? 2 : 4;
+    return p.b_dtype == DT_F16 && p.batch == 1 && (uint64_t)p.M * p.K * as < (1ull << 31) &&
+           (uint64_t)p.N * p.K * 2 < (1ull << 31) && (uint64_t)p.M * p.N < (1ull << 31) && p.K >= 32 && p.K < (1u << 22) &&
+           (!gated || p.H > 0);
+}
+
+// The tiles offered. A launch takes about 2.5 us plus, per round of tiles over
+// the CUs, `fixed` plus `chunk` per 64 k (us; index 0: fp16 X, 1: fp32 X;
+// measured on full grids at K = 768 and 2048).
+namespace ks {
+struct Tile { int bm, bn; float fixed[2], chunk[2]; };
+constexpr Tile TILES[] = {
+    {32, 32, {2.2f, 1.7f}, {.091f, .165f}},     // 8 waves split K
+    {32, 64, {2.2f, 2.3f}, {.14f, .18f}},       // 4 waves split K
+    {64, 64, {2.85f, 1.7f}, {.17f, .37f}},
+    {64, 128, {2.3f, 2.7f}, {.39f, .465f}},     // quadrants
+    {128, 128, {4.0f, 2.3f}, {.55f, .84f}},
+};
+constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
+
+// Whole 16-byte chunks everywhere: the copies go straight to LDS.
+inline bool dma_ok(const GemmParams& p)
+{
+    return p.K % 8 == 0 && ((uintptr_t)p.A % 16) == 0 && ((uintptr_t)p.B % 16) == 0;
+}
+}
+
+void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn)
+{
+    bm = ks::TILES[tile].bm;
+    bn = ks::TILES[tile].bn;
+}
+
+int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
+{
+    const int x = p.a_dtype == DT_F16 ? 0 : 1;
+    const float chunks = (float)((p.K + 63) / 64) * (ks::dma_ok(p) ? 1.f : 1.7f);   // (register staging: 1.5-1.9)
+    const uint32_t cols = gated ? 2 * p.H : p.N;
+    int best = 0;
+    *us = 1e30f;
+    for (int t = 0; t < ks::NTILES; ++t) {
+        const ks::Tile& k = ks::TILES[t];
+        const uint64_t tiles = (uint64_t)((p.M + k.bm - 1) / k.bm) * ((cols + k.bn - 1) / k.bn);
+        const float cost = 2.5f + (float)((tiles + cus - 1) / cus) * (k.fixed[x] + chunks * k.chunk[x]);
+        if (cost < *us) { *us = cost; best = t; }
+    }
+    return best;
+}
+
+template <typename C, bool GATED>
+static hipError_t launch_cfg(const GemmParams& p, hipStream_t s)
+{
+    static PerDevice lds_once;
+    hipError_t e = set_max_lds(lds_once, (const void*)gemm_ksplit_kernel<C, GATED>, C::LDS);
+    if (e != hipSuccess) return e;
+    const uint32_t no = GATED ? p.H : p.N, bno = GATED ? C::BN / 2 : C::BN;
+    const uint32_t tiles = ((p.M + C::BM - 1) / C::BM) * ((no + bno - 1) / bno) ;
+    hipLaunchKernelGGL((gemm_ksplit_kernel<C, GATED>), dim3(tiles), dim3(64 * C::NW), C::LDS, s, p);
+    return hipGetLastError();
+}
+
+template <typename TA, bool DMA, bool GATED>
+static hipError_t launch_tile(const GemmParams& p, int tile, hipStream_t s)
+{
+    constexpr bool H = sizeof(TA) == 2 || !DMA;   // X is fp16 in LDS
+    switch (tile) {
+    case 0: return launch_cfg<ks::Cfg<32, 32, 8, H ? 64 : 32, H ? 2 : 3, true, TA, DMA>, GATED>(p, s);
+    case 1: return launch_cfg<ks::Cfg<32, 64, 4, 64, H ? 3 : 2, true, TA, DMA>, GATED>(p, s);
+    case 2: return launch_cfg<ks::Cfg<64, 64, 4, H ? 64 : 32, H ? 2 : 3, true, TA, DMA>, GATED>(p, s);
+    case 3: return launch_cfg<ks::Cfg<64, 128, 4, 64, 4, false, TA, DMA>, GATED>(p, s);
+    case 4: return launch_cfg<ks::Cfg<128, 128, 4, 64, H ? 4 : 3, false, TA, DMA>, GATED>(p, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+template <typename TA, bool DMA>
+static hipError_t launch_gate(const GemmParams& p, bool gated, int tile, hipStream_t s)
+{
+    return gated ? launch_tile<TA, DMA, true>(p, tile, s) : launch_tile<TA, DMA, false>(p, tile, s);
+}
+
+hipError_t gemm_ksplit_launch(const GemmParams& p, bool gated, int tile, hipStream_t s)
+{
+    const bool dma = ks::dma_ok(p);
+    if (p.a_dtype == DT_F16)
+        return dma ? launch_gate<half_t, true>(p, gated, tile, s) : launch_gate<half_t, false>(p, gated, tile, s);
+    return dma ? launch_gate<float, true>(p, gated, tile, s) : launch_gate<float, false>(p, gated, tile, s);
+}
+
+}   // namespace vai_dev

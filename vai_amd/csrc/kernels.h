@@ -136,6 +136,14 @@ size_t gemm_packed_weight_bytes(uint32_t N, uint32_t K, uint32_t H, bool gated);
 hipError_t gemm_pack_weight(void* dst, const void* w, uint32_t N, uint32_t K, uint32_t H, bool gated, hipStream_t s);
 hipError_t gemm_packed_launch(const GemmParams& p, const void* packed, bool gated, hipStream_t s);
 
+// The sizes between: any fp16 weight as stored, fp16 or fp32 X, small tiles
+// whose waves split K (gemm_ksplit.hip). gemm_ksplit_plan returns the tile for
+// a launch and its modelled time.
+bool gemm_ksplit_ok(const GemmParams& p, bool gated);
+int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us);
+void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn);   // bn: logical columns (gated: gate and up)
+hipError_t gemm_ksplit_launch(const GemmParams& p, bool gated, int tile, hipStream_t s);
+
 // Linear with fp16 accumulation in the reference's exact fma order (any shape;
 // vector ALU, not the matrix cores, which accumulate in fp32 only).
 hipError_t gemm_acc16_launch(const GemmParams& p, bool gated, hipStream_t s);
