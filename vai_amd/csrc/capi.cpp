@@ -611,6 +611,16 @@ vai_status vai_conv2d_launch(const vai_conv2d_args* a, vai_stream_t stream)
         c.ks = a->kernel; c.stride = a->stride; c.epilogue = a->epilogue; c.residual_order = a->residual_order;
         return hip_status(conv_launch(c, a->i_dtype, (hipStream_t)stream));
     }
+    // rows and kernels the packed plan does not hold, over the weight as stored
+    if (a->w_dtype == VAI_DTYPE_F16 && conv_direct_ok(a->batch, a->ci, a->wi, a->co, ho, a->kernel, a->stride)) {
+        ConvDirectParams c{};
+        c.out = a->out; c.x = a->in; c.w = a->weight;
+        c.bias = a->bias; c.scale = a->scale; c.residual = a->residual;
+        c.o_dtype = a->o_dtype; c.residual_dtype = a->i_dtype;
+        c.batch = a->batch; c.ci = a->ci; c.hi = a->hi; c.wi = a->wi; c.co = a->co; c.ho = ho; c.wo = wo;
+        c.ks = a->kernel; c.stride = a->stride; c.epilogue = a->epilogue; c.residual_order = a->residual_order;
+        return hip_status(conv_direct_launch(c, a->i_dtype, (hipStream_t)stream));
+    }
     GemmParams g{};
     g.A = a->weight; g.B = a->in; g.C = a->out;
     g.a_dtype = a->w_dtype; g.b_dtype = a->i_dtype; g.c_dtype = a->o_dtype;

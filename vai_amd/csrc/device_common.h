@@ -166,4 +166,38 @@ __device__ __forceinline__ float swap_max32(float x)
     return fmaxf(x, y);
 }
 
+// 8 elements at any alignment, as fp16
+template <typename T>
+__device__ __forceinline__ half8 load8(const T* p)
+{
+    if constexpr (sizeof(T) == 2) {
+        typedef half8 half8u __attribute__((aligned(2)));
+        return *(const half8u*)p;
+    } else {
+        typedef float4v float4u __attribute__((aligned(4)));
+        const float4v lo = *(const float4u*)p, hi = *(const float4u*)(p + 4);
+        return __builtin_shufflevector(__builtin_convertvector(lo, half4), __builtin_convertvector(hi, half4), 0, 1, 2,
+                                       3, 4, 5, 6, 7);
+    }
+}
+
+// v moved down by s elements (0 .. 8), zeros from above
+__device__ __forceinline__ half8 shift_down(half8 v, uint32_t s)
+{
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 w = __builtin_bit_cast(u32x4, v);
+    const uint32_t d = s >> 1;
+    uint32_t x[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        x[i] = 0;
+#pragma unroll
+        for (int k = 0; k + i < 4; ++k) x[i] = d == (uint32_t)k ? w[i + k] : x[i];
+    }
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (s & 1) ? (x[i] >> 16) | (x[i + 1] << 16) : x[i];
+    return __builtin_bit_cast(half8, r);
+}
+
 }   // namespace vai_dev

@@ -267,6 +267,24 @@ hipError_t conv_pack_weight(half_t_storage* dst, const half_t_storage* w, uint32
                             hipStream_t s);
 hipError_t conv_launch(const ConvParams& p, int x_dt, hipStream_t s);
 
+// The same over the weight as stored, any image width and kernel
+// (conv_direct.hip).
+struct ConvDirectParams {
+    void* out;
+    const void* x;
+    const void* w;                // [Co][Ci][k][k] fp16
+    const void* bias;             // fp16 [Co] or null
+    const void* scale;            // fp16 [Co] or null
+    const void* residual;
+    int o_dtype, residual_dtype;
+    uint32_t batch, ci, hi, wi, co, ho, wo, ks, stride;
+    uint32_t epilogue, residual_order;
+    // set by the launch: channels per block, row tiles, multipliers for the kernel's divisions
+    uint32_t cb, ytiles, m_kk, m_c8, m_nv, m_wv;
+};
+bool conv_direct_ok(uint32_t batch, uint32_t ci, uint32_t wi, uint32_t co, uint32_t ho, uint32_t ks, uint32_t stride);
+hipError_t conv_direct_launch(ConvDirectParams p, int x_dt, hipStream_t s);
+
 // Split-K fold for Linear: O = s*epi(sum_z P[z] + B) (+R).
 hipError_t linear_reduce_launch(void* out, int o_dtype, const float* partials, uint32_t splits, size_t MN,
                                 const void* bias, int b_dtype, uint32_t bias_repeat,
