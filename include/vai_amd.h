@@ -86,9 +86,9 @@ typedef struct {
     uint32_t split_size;
     uint32_t gated;
     uint32_t gate_epilogue;
-    /* NULL, or vai_linear_pack_weight()'s output for this weight: prefill
-     * shapes (M > 8, fp16 I and W) then stream W into the matrix cores from
-     * that fragment-major copy instead of staging it through LDS. */
+    /* NULL, or vai_linear_pack_weight()'s output for this weight: fp16 I and W
+     * with M >= 3 then read W from that fragment-major copy (M of 512 and more
+     * straight into the matrix cores' registers). */
     const void* packed_weight;
     /* Accumulator dtype, Linear::setAccDtype (/root/reference/vai/nodes/
      * linear.h:289,2320): VAI_DTYPE_F32 (0, the default and the reference's

@@ -86,3 +86,31 @@ def test_ksplit_gated(gpu, m, k, h, xdt, odt, tile):
 def test_ksplit_unaligned_weight(gpu):
     """A weight two bytes off a 16-byte boundary is staged through registers."""
     check(gpu, 20, 512, 64, F16, F32, "32x32", off=1)
+
+
+@pytest.mark.parametrize("m, k, n, gated, tile", [
+    (9, 256, 33, False, "32x32"), (61, 3072, 5120, False, "32x64"), (100, 1024, 5000, False, "64x64"),
+    (300, 512, 4100, False, "64x128"), (400, 384, 8192, False, "128x128"),
+    (9, 256, 34, True, "32x32"), (40, 1024, 4100, True, "32x64"), (300, 512, 4200, True, "64x128"),
+])
+def test_ksplit_packed_weight(gpu, m, k, n, gated, tile):
+    """The packed weight takes the same k order: the same bits, from the packed
+    copy alone (the weight it was packed from is overwritten with NaNs)."""
+    rng = np.random.default_rng(n)
+    D = gpu.DeviceArray.from_numpy
+    dw, dx = D(draw(normal((n, k), 0.05), rng, F16)), D(draw((m, k), rng, F16))
+    outs = [gpu.DeviceArray((m, n // 2 if gated else n), F32) for _ in range(2)]
+    for i, out in enumerate(outs):
+        out.fill_(0xFF)
+        a = gpu.linear_args(out, dx, dw, None, None, gated=gated, gate_epi="SILU")
+        if i:
+            packed = gpu.linear_pack_weight(a)
+            a.packed_weight = packed.ptr
+            dw.fill_(0xFF)
+        name = gpu.linear_plan(a)[0]
+        print(f"ksplit packed={i} m={m} k={k} n={n} gated={gated} plan={name}", flush=True)
+        assert name == f"tile_f16_{tile}_kwaves" + ("_gated" if gated else "")
+        gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
+        gpu.synchronize()
+    got, want = outs[1].numpy(), outs[0].numpy()
+    assert np.isfinite(got).all() and (got == want).all()

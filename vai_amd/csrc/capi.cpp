@@ -371,7 +371,9 @@ static vai_status linear_run(const vai_linear_args* a, const LinearPlan& p, hipS
                                                a->gate_epilogue, a->N, s));
     }
     if (p.kind == LinearPlan::F32Small) return hip_status(gemm_f32_launch(g, (int)(p.bn / 16), s));
-    hipError_t e = p.kind == LinearPlan::KSplit ? gemm_ksplit_launch(g, a->gated != 0, p.ks_tile, s) : gemm_launch(g, a->gated ? BKind::Gated : BKind::Dense,
+    if (p.kind == LinearPlan::KSplit)
+        return hip_status(gemm_ksplit_launch(g, linear_packable(a) ? a->packed_weight : nullptr, a->gated != 0, p.ks_tile, s));
+    hipError_t e = gemm_launch(g, a->gated ? BKind::Gated : BKind::Dense,
                                a->gated ? EpiKind::Gated : EpiKind::Linear, p.tile, s);
     if (e != hipSuccess || p.splits == 1) return hip_status(e);
     const size_t MN = (size_t)a->M * (a->gated ? a->N / 2 : a->N);

@@ -48,11 +48,14 @@ namespace ks {
 // One variant: tile, waves, k per stage and ring depth for X of type TA.
 // KSP: the waves split K, each with its own ring; otherwise four waves take a
 // quadrant each of the tile and share one ring. DMA false: staged through
-// registers (one stage per wave, or two shared ones), X in LDS as fp16.
-template <int BM_, int BN_, int NW_, int BK_, int S_, bool KSP_, typename TA_, bool DMA_>
+// registers (one stage per wave, or two shared ones), X in LDS as fp16. PK:
+// the weight is gemm_pack_weight's copy, whose 16-byte pieces (8 k of one row,
+// 32 rows of a block after each other) are staged in that order: whole
+// contiguous copies, and fragment reads of 1 KB without a swizzle.
+template <int BM_, int BN_, int NW_, int BK_, int S_, bool KSP_, typename TA_, bool DMA_, bool PK_>
 struct Cfg {
     static constexpr int BM = BM_, BN = BN_, NW = NW_, BK = BK_, S = DMA_ ? S_ : (KSP_ ? 1 : 2);
-    static constexpr bool KSP = KSP_, DMA = DMA_;
+    static constexpr bool KSP = KSP_, DMA = DMA_, PK = PK_;
     typedef TA_ TA;
     static constexpr int WM = KSP ? BM : BM / 2, WN = KSP ? BN : BN / 2;   // a wave's part of the tile
     // sums per output and wave (k steps in turn)
@@ -94,7 +97,7 @@ __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 
 }   // namespace ks
 
 template <typename C, bool GATED>
-__global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_kernel(GemmParams p)
+__global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_kernel(GemmParams p, const half_t* __restrict__ packed)
 {
     using namespace ks;
     constexpr int BM = C::BM, BN = C::BN, NW = C::NW, BK = C::BK, S = C::S;
@@ -153,8 +156,16 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
         ra = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(A + (size_t)m0 * K), (short)0,
                                                (int)__builtin_amdgcn_readfirstlane((M - m0) * K * (uint32_t)sizeof(TA)),
                                                0x00020000);
-        rb = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)uniform_ptr(B), (short)0, (int)__builtin_amdgcn_readfirstlane((GATED ? 2 * H : N) * K * 2), 0x00020000);
+        // packed: the tile's 32-row blocks from block nb0 on (a block is K * 64
+        // bytes; padding blocks fill the tile), the k steps by scalar offset
+        const uint32_t nb0 = GATED ? n0 / 32 * 2 : n0 / 32;
+        if constexpr (C::PK)
+            rb = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(packed + (size_t)nb0 * K * 32), (short)0,
+                                                   (int)__builtin_amdgcn_readfirstlane((GATED && BN < 64 ? 2 : BN / 32) * K * 64),
+                                                   0x00020000);
+        else
+            rb = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(B), (short)0,
+                                                   (int)__builtin_amdgcn_readfirstlane((GATED ? 2 * H : N) * K * 2), 0x00020000);
 #pragma unroll
         for (int i = 0; i < C::ACOPIES; ++i) {
             const int s = (cw * C::ACOPIES + i) * 64 + lane, row = s / ACH, ch = swz<C::AROW>(row, s % ACH);
@@ -162,8 +173,17 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
         }
 #pragma unroll
         for (int i = 0; i < C::BCOPIES; ++i) {
-            const int s = (cw * C::BCOPIES + i) * 64 + lane, row = s / BCH, ch = swz<C::BROW>(row, s % BCH);
-            boff[i] = (wrow(row) * K + ch * 8) * 2;
+            const int s = (cw * C::BCOPIES + i) * 64 + lane;
+            if constexpr (C::PK) {
+                // slot s: chunk s / BN, tile column s % BN
+                const uint32_t ch = s / BN, j = s % BN;
+                const uint32_t jo = GATED ? n0 % 32 + (j < (uint32_t)BNO ? j : j - BNO) : j;   // row within the tile's blocks
+                const uint32_t blk = GATED ? jo / 32 * 2 + (j < (uint32_t)BNO ? 0 : 1) : jo / 32;
+                boff[i] = blk * K * 64 + (ch * 32 + jo % 32) * 16;
+            } else {
+                const int row = s / BCH, ch = swz<C::BROW>(row, s % BCH);
+                boff[i] = (wrow(row) * K + ch * 8) * 2;
+            }
         }
     }
     // Part q of KSTEPS of this wave's copies of chunk c into a slot, spread over
@@ -184,10 +204,10 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
         }
 #pragma unroll
         for (int i = C::BCOPIES * q / KSTEPS; i < C::BCOPIES * (q + 1) / KSTEPS; ++i) {
-            const int s = (cw * C::BCOPIES + i) * 64 + lane, ch = swz<C::BROW>(s / BCH, s % BCH);
+            const int s = (cw * C::BCOPIES + i) * 64 + lane, ch = C::PK ? s / BN : swz<C::BROW>(s / BCH, s % BCH);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_AS void*)(bdst + i * 1024), 16,
                                                      (int)((uint32_t)ch * 8 < left ? boff[i] : 0x80000000u),
-                                                     (int)(k0 * 2), 0, 0);
+                                                     (int)(k0 * (C::PK ? 64 : 2)), 0, 0);
         }
     };
     const auto issue = [&](int slot, int c) __attribute__((always_inline)) {
@@ -253,6 +273,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     };
     const auto read_w = [&](const LDS_AS char* st, int j, int q) __attribute__((always_inline)) {
         const int row = wn0 + j * 32 + fr;
+        if constexpr (C::PK) return *(const LDS_AS half8*)(st + C::ABYTES + ((q * 2 + fk) * BN + row) * 16);
         return *(const LDS_AS half8*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, q * 2 + fk) * 16);
     };
 
@@ -559,43 +580,50 @@ int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
 }
 
 template <typename C, bool GATED>
-static hipError_t launch_cfg(const GemmParams& p, hipStream_t s)
+static hipError_t launch_cfg(const GemmParams& p, const void* packed, hipStream_t s)
 {
     static PerDevice lds_once;
     hipError_t e = set_max_lds(lds_once, (const void*)gemm_ksplit_kernel<C, GATED>, C::LDS);
     if (e != hipSuccess) return e;
     const uint32_t no = GATED ? p.H : p.N, bno = GATED ? C::BN / 2 : C::BN;
     const uint32_t tiles = ((p.M + C::BM - 1) / C::BM) * ((no + bno - 1) / bno) ;
-    hipLaunchKernelGGL((gemm_ksplit_kernel<C, GATED>), dim3(tiles), dim3(64 * C::NW), C::LDS, s, p);
+    hipLaunchKernelGGL((gemm_ksplit_kernel<C, GATED>), dim3(tiles), dim3(64 * C::NW), C::LDS, s, p, (const half_t*)packed);
     return hipGetLastError();
 }
 
-template <typename TA, bool DMA, bool GATED>
-static hipError_t launch_tile(const GemmParams& p, int tile, hipStream_t s)
+template <typename TA, bool DMA, bool PK, bool GATED>
+static hipError_t launch_tile(const GemmParams& p, const void* packed, int tile, hipStream_t s)
 {
     constexpr bool H = sizeof(TA) == 2 || !DMA;   // X is fp16 in LDS
     switch (tile) {
-    case 0: return launch_cfg<ks::Cfg<32, 32, 8, H ? 64 : 32, H ? 2 : 3, true, TA, DMA>, GATED>(p, s);
-    case 1: return launch_cfg<ks::Cfg<32, 64, 4, 64, H ? 3 : 2, true, TA, DMA>, GATED>(p, s);
-    case 2: return launch_cfg<ks::Cfg<64, 64, 4, H ? 64 : 32, H ? 2 : 3, true, TA, DMA>, GATED>(p, s);
-    case 3: return launch_cfg<ks::Cfg<64, 128, 4, 64, 4, false, TA, DMA>, GATED>(p, s);
-    case 4: return launch_cfg<ks::Cfg<128, 128, 4, 64, H ? 4 : 3, false, TA, DMA>, GATED>(p, s);
+    case 0: return launch_cfg<ks::Cfg<32, 32, 8, H ? 64 : 32, H ? 2 : 3, true, TA, DMA, PK>, GATED>(p, packed, s);
+    case 1: return launch_cfg<ks::Cfg<32, 64, 4, 64, H ? 3 : 2, true, TA, DMA, PK>, GATED>(p, packed, s);
+    case 2: return launch_cfg<ks::Cfg<64, 64, 4, H ? 64 : 32, H ? 2 : 3, true, TA, DMA, PK>, GATED>(p, packed, s);
+    case 3: return launch_cfg<ks::Cfg<64, 128, 4, 64, 4, false, TA, DMA, PK>, GATED>(p, packed, s);
+    case 4: return launch_cfg<ks::Cfg<128, 128, 4, 64, H ? 4 : 3, false, TA, DMA, PK>, GATED>(p, packed, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-template <typename TA, bool DMA>
-static hipError_t launch_gate(const GemmParams& p, bool gated, int tile, hipStream_t s)
+template <typename TA, bool DMA, bool PK>
+static hipError_t launch_gate(const GemmParams& p, const void* packed, bool gated, int tile, hipStream_t s)
 {
-    return gated ? launch_tile<TA, DMA, true>(p, tile, s) : launch_tile<TA, DMA, false>(p, tile, s);
+    return gated ? launch_tile<TA, DMA, PK, true>(p, packed, tile, s) : launch_tile<TA, DMA, PK, false>(p, packed, tile, s);
 }
 
-hipError_t gemm_ksplit_launch(const GemmParams& p, bool gated, int tile, hipStream_t s)
+hipError_t gemm_ksplit_launch(const GemmParams& p, const void* packed, bool gated, int tile, hipStream_t s)
 {
     const bool dma = ks::dma_ok(p);
-    if (p.a_dtype == DT_F16)
-        return dma ? launch_gate<half_t, true>(p, gated, tile, s) : launch_gate<half_t, false>(p, gated, tile, s);
-    return dma ? launch_gate<float, true>(p, gated, tile, s) : launch_gate<float, false>(p, gated, tile, s);
+    if (p.a_dtype == DT_F16) {
+        // (the packed form has K % 128 == 0: no short chunk). The weight itself
+        // is then not read, as in the 256x256 kernel over the packed form.
+        if (packed && ((uintptr_t)packed % 16) == 0 && ((uintptr_t)p.A % 16) == 0)
+            return launch_gate<half_t, true, true>(p, packed, gated, tile, s);
+        return dma ? launch_gate<half_t, true, false>(p, nullptr, gated, tile, s)
+                   : launch_gate<half_t, false, false>(p, nullptr, gated, tile, s);
+    }
+    return dma ? launch_gate<float, true, false>(p, nullptr, gated, tile, s)
+               : launch_gate<float, false, false>(p, nullptr, gated, tile, s);
 }
 
 }   // namespace vai_dev

@@ -142,7 +142,8 @@ hipError_t gemm_packed_launch(const GemmParams& p, const void* packed, bool gate
 bool gemm_ksplit_ok(const GemmParams& p, bool gated);
 int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us);
 void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn);   // bn: logical columns (gated: gate and up)
-hipError_t gemm_ksplit_launch(const GemmParams& p, bool gated, int tile, hipStream_t s);
+// packed: null, or gemm_pack_weight's copy of an fp16 weight for fp16 X
+hipError_t gemm_ksplit_launch(const GemmParams& p, const void* packed, bool gated, int tile, hipStream_t s);
 
 // Linear with fp16 accumulation in the reference's exact fma order (any shape;
 // vector ALU, not the matrix cores, which accumulate in fp32 only).
