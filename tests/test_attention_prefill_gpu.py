@@ -1,0 +1,56 @@
+"""Prefill attention at the edges of its workgroup order and tiles, against
+float64. Bound, with A = sum p |v| of the row: P is rounded to fp16 (2^-11 A), a
+score's D products are summed in fp32 (D 2^-24 sum |q k| scale, which moves p
+and 1 / l by that much each), exp2 and the sums over keys (32 + T / 64 steps of
+2^-24 each side), and the output rounding."""
+import numpy as np
+import pytest
+
+from helpers import draw
+
+pytestmark = pytest.mark.gpu
+F16, F32 = np.float16, np.float32
+
+
+@pytest.mark.parametrize("b, hq, hkv, tq, tkv, d, causal, span, odt", [
+    (1, 256, 32, 130, 130, 64, True, 0, F32),      # a multiple of 8 pairs, unsplit, two query tiles
+    (2, 132, 44, 129, 129, 64, True, 0, F16),      # 264 pairs of two batches
+    (1, 150, 50, 300, 300, 128, True, 0, F16),     # pairs not a multiple of 8: heads spread over the XCDs
+    (1, 131, 131, 257, 200, 128, True, 0, F32),    # rows that see no key
+    (1, 90, 30, 385, 450, 128, False, 0, F32),     # no mask, a key tail of two rows
+    (1, 72, 24, 520, 520, 80, True, 70, F16),      # window, padded head dim
+    (3, 43, 43, 300, 300, 256, True, 0, F32),
+    (1, 24, 8, 1000, 1000, 128, True, 0, F32),     # fewer tiles than CUs: split
+    (1, 16, 2, 256, 2111, 128, True, 0, F16),      # long walks, an odd number of tiles
+    (1, 4, 4, 64, 65, 64, False, 0, F32),
+    (1, 2, 2, 100, 64, 128, False, 0, F16),        # one key tile
+])
+def test_prefill(gpu, b, hq, hkv, tq, tkv, d, causal, span, odt):
+    rng = np.random.default_rng(tq + d + hq)
+    q, k, v = (draw((b, h, t, d), rng, F16) for h, t in ((hq, tq), (hkv, tkv), (hkv, tkv)))
+    D = gpu.DeviceArray.from_numpy
+    out = gpu.DeviceArray((b, tq, hq, d), odt)
+    out.fill_(0xFF)
+    print(f"prefill b={b} hq={hq} hkv={hkv} tq={tq} tkv={tkv} d={d} causal={causal} span={span}", flush=True)
+    got = gpu.attention(out, D(q), D(k), D(v), causal=causal, span=span).numpy().astype(np.float64)
+    i, j = np.arange(tq)[:, None] + (tkv - tq), np.arange(tkv)[None, :]
+    vis = (j <= i) if causal else np.ones((tq, tkv), bool)
+    if span:
+        vis = vis & (j > i - span)
+    none = ~vis.any(axis=1)
+    e = 2.0 ** -24
+    for bb in range(b):
+        for h in list(range(0, hq, max(1, hq // 9))) + [hq - 1]:
+            q64, k64, v64 = (x.astype(np.float64) for x in (q[bb, h], k[bb, h // (hq // hkv)], v[bb, h // (hq // hkv)]))
+            s = np.where(vis, q64 @ k64.T / np.sqrt(d), -np.inf)
+            mx = np.where(none, 0.0, s.max(axis=1, initial=-np.inf))
+            p = np.exp(s - mx[:, None])
+            p /= np.maximum(p.sum(axis=1, keepdims=True), 1e-300)
+            y, A = p @ v64, p @ np.abs(v64)
+            err = d * e * (np.abs(q64) @ np.abs(k64).T / np.sqrt(d)).max() + (32 + tkv / 64 + 8) * e
+            tol = A * (2.0 ** -11 + 2 * err) + (2.0 ** -11 * np.abs(y) if odt == F16 else 0) + 2.0 ** -24
+            if odt == F16 and tkv > 64:
+                tol = tol + 2.0 ** -10 * A       # split walks: partials rounded to fp16 before they are merged
+            r = got[bb, :, h]
+            assert np.isfinite(r).all() and (np.abs(r - y) <= tol).all(), (h, float((np.abs(r - y) / tol).max()))
+            assert (r[none] == 0).all()

@@ -21,8 +21,8 @@
 //    read from V's row-major LDS tile with ds_read_b64_tr_b16 (4 keys of one
 //    column per lane per read) in the key order the P^T registers hold. O^T
 //    gives lane l query l % 32 again, so the per-row rescale and the final
-//    1/l use the lane's own m and l. O^T lives in accumulation registers,
-//    D/32 fragments of 32x32.
+//    1/l use the lane's own m and l. O^T lives in registers (accumulation
+//    registers at D = 256), D/32 fragments of 32x32.
 //  * K and V tiles (row-major, 16-byte chunks XOR-swizzled by row) are copied
 //    global -> LDS by buffer_load ... lds, double buffered: the copies of tile
 //    t + 1 are issued during tile t's S^T MFMAs, a few per MFMA group (issued
@@ -111,22 +111,13 @@ __device__ __forceinline__ float fa_scale_acc(float x, float a)
     return x;
 }
 
-// Pairwise tree reductions of 32 values (depth 5 instead of a chain of 31).
-__device__ __forceinline__ float fa_tree_max(float (&v)[32])
+// Maximum of three (fmaxf keeps a quieting v_max per operand that comes from a
+// matrix core: 46 instructions for a tile's 32 scores instead of 16).
+__device__ __forceinline__ float fa_max3(float a, float b, float c)
 {
-#pragma unroll
-    for (int w = 16; w >= 1; w >>= 1)
-#pragma unroll
-        for (int i = 0; i < w; ++i) v[i] = fmaxf(v[i], v[i + w]);
-    return v[0];
-}
-__device__ __forceinline__ float fa_tree_sum(float (&v)[32])
-{
-#pragma unroll
-    for (int w = 16; w >= 1; w >>= 1)
-#pragma unroll
-        for (int i = 0; i < w; ++i) v[i] += v[i + w];
-    return v[0];
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
 }
 
 template <int N>
@@ -238,8 +229,17 @@ __device__ __forceinline__ void fa_wait_vmcnt()
 // 256); HD = p.head_dim <= D is the operands' own, a multiple of 8. The
 // padding reads as zero (out of the buffers' range), so it adds nothing to
 // any score or output; output columns past HD are not stored.
+//
+// A wave alternates between matrix-core phases (S^T, P.V) and the softmax, so
+// one wave per SIMD leaves each unit idle during the other's phase. D <= 128
+// keeps to 256 registers (O in ordinary registers, K fragments four at a time,
+// the softmax eight scores at a time): two workgroups per CU, one's softmax
+// under the other's MFMAs (D = 64: three). Causal 24 x 4096 x 128 heads: 224 us
+// with one wave per SIMD and each head's walks in turn, 122 us now, 840 TFLOP/s
+// of visible work; the LDS fragment reads (128 KB a tile and workgroup) bound it
+// next. D = 256 needs 392 registers and 128 KB: one workgroup per CU.
 template <int D>
-__global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
+__global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention_fwd_kernel(AttnParams p)
 {
     using namespace fa;
     using L = Lds<D>;
@@ -272,13 +272,18 @@ __global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
         h = (e1 >> 10) & 0x3FF;
         b = e1 >> 20;
     } else {
-        // Workgroup -> (query tile, head, batch) with one head's query
-        // tiles on one XCD (fa_xcd_block), the longest causal walks first.
-        const uint32_t X = gridDim.x, HX = X * gridDim.y;
-        const uint32_t lb = fa_xcd_block(blockIdx.x + X * (blockIdx.y + gridDim.y * blockIdx.z), HX * gridDim.z);
-        unit = lb % X;
-        h = (lb / X) % gridDim.y;
-        b = lb / HX;
+        // Workgroup -> (query tile, head, batch): the longest causal walks of
+        // all heads first, so that the short ones fill the end; linear
+        // workgroup w runs on XCD w % 8, so with a multiple of 8 (head, batch)
+        // pairs each XCD takes whole neighbouring heads (one K / V of a group).
+        // (Head by head, the last head's longest walk starts when the chip runs
+        // dry: 130 tiles on the busiest CU where the average is 99.)
+        const uint32_t X = gridDim.x, P = gridDim.y * gridDim.z;
+        const uint32_t w = blockIdx.x + X * (blockIdx.y + gridDim.y * blockIdx.z);
+        const uint32_t pr = w % P, hb = P % 8 == 0 ? pr % 8 * (P / 8) + pr / 8 : pr;
+        unit = w / P;
+        h = hb % gridDim.y;
+        b = hb / gridDim.y;
         qt = nqt - 1 - unit;
     }
     qt = __builtin_amdgcn_readfirstlane(qt);
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
         // key block i % 2, head-dim step i / 2 (two independent accumulation
         // chains); K fragments are read in groups of G, the next group's
         // reads in flight behind the current group's MFMAs.
-        constexpr int NS = 2 * KS, G = NS < 8 ? NS : (D == 256 ? 4 : 8);
+        constexpr int NS = 2 * KS, G = D == 64 ? 8 : 4;
         constexpr int OPG = 2 * L::COPIES / (NS / G);   // tile t + 1 copies per MFMA group
         static_assert(OPG * (NS / G) == 2 * L::COPIES, "copies spread evenly over the groups");
         const bool next = t + 1 < ntiles;
@@ -460,15 +465,8 @@ __global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
         // scale take the short path: the max over the raw scores, then
         // 2^(fma(s, scale', -m)). Others scale and mask first.
         const bool fast = __all(j0 >= row_kbeg && j0 + BKV <= row_kend) && sl2 >= 0.f;
-        // (reductions as trees: with one wave per SIMD a chain of dependent
-        // steps costs its whole latency)
-        float tv[32];
-        float tmax;
-        if (fast) {
-#pragma unroll
-            for (int i = 0; i < 32; ++i) tv[i] = sacc[i >> 4][i & 15];
-            tmax = fa_tree_max(tv) * sl2;
-        } else {
+        // (reductions as trees, not chains of dependent steps)
+        if (!fast) {
             // visible local keys [lo, hi) of the tile, clamped into [-1, 65]
             const int lo = (int)std::min<int64_t>(std::max<int64_t>(row_kbeg - j0, -1), 65);
             const int hi = (int)std::min<int64_t>(std::max<int64_t>(row_kend - j0, -1), 65);
@@ -477,12 +475,16 @@ __global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
 #pragma unroll
                 for (int rr = 0; rr < 16; ++rr) {
                     const int kl = kb * 32 + 8 * (rr >> 2) + 4 * hf + (rr & 3);
-                    const float v = (kl >= hi || kl < lo) ? -__builtin_inff() : sacc[kb][rr] * sl2;
-                    sacc[kb][rr] = v;
-                    tv[kb * 16 + rr] = v;
+                    sacc[kb][rr] = (kl >= hi || kl < lo) ? -__builtin_inff() : sacc[kb][rr] * sl2;
                 }
-            tmax = fa_tree_max(tv);
         }
+        float tm[10];
+#pragma unroll
+        for (int i = 0, j = 0; i < 10; ++i, j += 3)
+            tm[i] = fa_max3(sacc[j >> 4][j & 15], sacc[(j + 1) >> 4][(j + 1) & 15], sacc[(j + 2) >> 4][(j + 2) & 15]);
+        float tmax = fa_max3(fa_max3(tm[0], tm[1], tm[2]), fa_max3(tm[3], tm[4], tm[5]),
+                             fa_max3(fa_max3(tm[6], tm[7], tm[8]), tm[9], fa_max3(sacc[1][14], sacc[1][15], sacc[1][15])));
+        if (fast) tmax *= sl2;
         tmax = swap_max32(tmax);
         // Lazy rescaling: the reference m of a row (the exponent offset of
         // its O and l) moves only when the row max exceeds it by more than
@@ -502,33 +504,28 @@ __global__ __launch_bounds__(256, 1) void attention_fwd_kernel(AttnParams p)
 #pragma unroll
                 for (int d = 0; d < DF; ++d)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) o[d][r] = fa_scale_acc(o[d][r], alpha);
+                    for (int r = 0; r < 16; ++r) {
+                        if constexpr (D == 256) o[d][r] = fa_scale_acc(o[d][r], alpha);
+                        else o[d][r] *= alpha;
+                    }
             }
         }
         const float mref = m == -__builtin_inff() ? 0.f : m;
         half8 pb[4];   // P^T operand of key step kk: registers 8 (kk % 2) .. +7 of block kk / 2
-        if (fast) {
+        const float esc = fast ? sl2 : 1.f;
+        float ps[4];
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+        for (int kk = 0; kk < 4; ++kk) {
+            float8v e;
 #pragma unroll
-                for (int rr = 0; rr < 16; ++rr) {
-                    const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][rr], sl2, -mref));
-                    tv[kb * 16 + rr] = e;
-                    pb[2 * kb + (rr >> 3)][rr & 7] = (half_t)e;
-                }
-        } else {
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int rr = 0; rr < 16; ++rr) {
-                    const float e = __builtin_amdgcn_exp2f(sacc[kb][rr] - mref);
-                    tv[kb * 16 + rr] = e;
-                    pb[2 * kb + (rr >> 3)][rr & 7] = (half_t)e;
-                }
+            for (int i = 0; i < 8; ++i)
+                e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kk >> 1][8 * (kk & 1) + i], esc, -mref));
+            pb[kk] = __builtin_convertvector(e, half8);
+            ps[kk] = ((e[0] + e[4]) + (e[1] + e[5])) + ((e[2] + e[6]) + (e[3] + e[7]));
         }
         {
-            const float ps = fa_tree_sum(tv);
-            l += swap_sum<32>(ps, ps);
+            const float pt = (ps[0] + ps[2]) + (ps[1] + ps[3]);
+            l += swap_sum<32>(pt, pt);
         }
 
         // O^T += V^T P^T over the tile's four 16-key steps, the next step's
