@@ -1,7 +1,8 @@
 """The small-tile Linear (gemm_ksplit.hip) against float64, at the edges of its
 tiles, k chunks and both staging forms. The bound is the rounding an fp32 sum
-of K exact products can make, K 2^-24 sum |x w|, plus one fp16 rounding of each
-fp32 activation (2^-11 sum |x w|) and of the output (2^-11 |y|)."""
+of K products can make, (K + 1) 2^-24 sum |x w|, plus one fp16 rounding of each
+fp32 activation that meets fp16 weights (2^-11 sum |x w|) and of the output
+(2^-11 |y|)."""
 import ctypes
 
 import numpy as np
@@ -17,27 +18,27 @@ def silu(v):
     return v / (1 + np.exp(-v))
 
 
-def check(gpu, m, k, n, xdt, odt, tile, bias=None, residual=None, gated=False, off=0):
+def check(gpu, m, k, n, xdt, odt, tile, bias=None, residual=None, gated=False, off=0, wdt=F16):
     rng = np.random.default_rng(m + k + n)
-    w, x = draw(normal((n, k), 0.05), rng, F16), draw((m, k), rng, xdt)
+    w, x = draw(normal((n, k), 0.05), rng, wdt), draw((m, k), rng, xdt)
     b = draw(normal((n,) if bias == "row" else (m, n), 0.05), rng, F16) if bias else None
     r = draw((n,) if residual == "row" else (m, n), rng, odt) if residual else None
     D = gpu.DeviceArray.from_numpy
-    dw = D(np.concatenate([np.zeros(off, F16), w.ravel()]))
+    dw = D(np.concatenate([np.zeros(off, wdt), w.ravel()]))
     dx, db, dr = D(x), None if b is None else D(b), None if r is None else D(r)
     out = gpu.DeviceArray((m, n // 2 if gated else n), odt)
     out.fill_(0xFF)
     a = gpu.linear_args(out, dx, D(w), db, dr, gated=gated, gate_epi="SILU")
-    a.weight = dw.ptr + 2 * off
+    a.weight = dw.ptr + w.itemsize * off
     name, splits = gpu.linear_plan(a)
     print(f"ksplit m={m} k={k} n={n} {np.dtype(xdt)} -> {np.dtype(odt)} gated={gated} plan={name}", flush=True)
-    assert name == f"tile_f16_{tile}_kwaves" + ("_gated" if gated else "") and splits == 1
+    assert name == f"tile_f{8 * w.itemsize}_{tile}_kwaves" + ("_gated" if gated else "") and splits == 1
     assert gpu.lib().vai_linear_workspace_size(ctypes.byref(a)) == 0
     gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
     gpu.synchronize()
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     mag = np.abs(x64) @ np.abs(w64).T
-    tol = mag * (k * 2.0 ** -24 + (2.0 ** -11 if xdt == F32 else 0)) + 1e-6
+    tol = mag * ((k + 1) * 2.0 ** -24 + (2.0 ** -11 if xdt == F32 and wdt == F16 else 0)) + 1e-6
     y = x64 @ w64.T + (0 if b is None else b.astype(np.float64))
     if gated:
         h = n // 2
@@ -81,6 +82,19 @@ def test_ksplit(gpu, m, k, n, xdt, odt, tile, kw):
 ])
 def test_ksplit_gated(gpu, m, k, h, xdt, odt, tile):
     check(gpu, m, k, 2 * h, xdt, odt, tile, bias="row", gated=True)
+
+
+@pytest.mark.parametrize("m, k, n, odt, tile, kw", [
+    (1024, 768, 3072, F32, "64x64", {"bias": "row"}),          # whole tiles
+    (1000, 100, 3201, F16, "64x64", {"residual": "full"}),     # a short last chunk, one column past a tile
+    (900, 301, 3100, F32, "64x64", {"bias": "full"}),         # odd K: through registers
+    (9, 33, 40, F32, "32x32", {}),                            # two chunks for eight waves, the second of one k
+    (33, 1147, 96, F16, "32x32", {"bias": "row", "residual": "row"}),
+    (70, 1028, 1000, F32, "32x32", {"residual": "full"}),     # K % 4 == 0: direct copies, a short last chunk
+    (64, 516, 64, F32, "32x32", {"off": 1}),                  # W off a 16-byte boundary
+])
+def test_ksplit_f32(gpu, m, k, n, odt, tile, kw):
+    check(gpu, m, k, n, F32, odt, tile, wdt=F32, **kw)
 
 
 def test_ksplit_unaligned_weight(gpu):

@@ -187,10 +187,14 @@ LinearPlan plan_linear(const vai_linear_args* a)
             }
             g.splits = 1;
         }
-        // fp32 problems with fewer 64x64 tiles than CUs: one launch over the
-        // full K with a CU-filling tile count, instead of split-K + reduce
-        if (a->split_size == 0 && !a->gated && gemm_f32_ok(g) && tiles_of(M, N, 64, 64) < plan_cus()) {
-            const int nf = gemm_f32_nf(M, N, plan_cus());
+        // fp32 problems with fewer 64x64 tiles than CUs, or where its rounds of
+        // 32-row tiles still take less: one launch over the full K with a
+        // CU-filling tile count
+        const int nf = gemm_f32_nf(M, N, plan_cus());
+        const float f32_us = 2.5f + (float)((tiles_of(M, N, 32, 16 * nf) + plan_cus() - 1) / plan_cus()) *
+                                        (2.f + 0.0022f * (float)nf * (float)K);
+        if (a->split_size == 0 && !a->gated && gemm_f32_ok(g) &&
+            (tiles_of(M, N, 64, 64) < plan_cus() || !ksplit || f32_us <= ksplit_us)) {
             p.kind = LinearPlan::F32Small;
             p.bm = 32;
             p.bn = 16 * nf;
@@ -301,7 +305,8 @@ vai_status vai_linear_plan(const vai_linear_args* a, char* name, size_t name_len
     } else if (p.kind == LinearPlan::KSplit) {
         uint32_t bm, bn;
         gemm_ksplit_tile(p.ks_tile, bm, bn);
-        snprintf(buf, sizeof buf, "tile_f16_%ux%u_kwaves%s", bm, bn, a->gated ? "_gated" : "");
+        snprintf(buf, sizeof buf, "tile_f%d_%ux%u_kwaves%s", a->w_dtype == VAI_DTYPE_F16 ? 16 : 32, bm, bn,
+                 a->gated ? "_gated" : "");
     } else {
         const bool f32 = a->i_dtype == VAI_DTYPE_F32 && a->w_dtype == VAI_DTYPE_F32;
         snprintf(buf, sizeof buf, "tile_%s_%s%s", f32 ? "f32" : "f16", tile_name(p.tile, a->gated),

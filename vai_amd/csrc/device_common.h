@@ -181,6 +181,24 @@ __device__ __forceinline__ half8 load8(const T* p)
     }
 }
 
+// 4 consecutive floats at any 4-byte address, and v moved down by s elements
+__device__ __forceinline__ float4v load4f(const float* p)
+{
+    typedef float4v float4u __attribute__((aligned(4)));
+    return *(const float4u*)p;
+}
+__device__ __forceinline__ float4v shift_down(float4v v, uint32_t s)
+{
+    float4v r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        r[i] = 0.f;
+#pragma unroll
+        for (int k = 0; k + i < 4; ++k) r[i] = s == (uint32_t)k ? v[i + k] : r[i];
+    }
+    return r;
+}
+
 // v moved down by s elements (0 .. 8), zeros from above
 __device__ __forceinline__ half8 shift_down(half8 v, uint32_t s)
 {

@@ -29,7 +29,14 @@
 // N 1216 (odd K) 205 -> 28; gated fp16 [500, 2048], H 2048 71 -> 16. At 32x32
 // a workgroup moves 8.7 us per MB of its operands, 50 bytes a cycle.
 //
-// Rows that are not whole 16-byte chunks (K % 8 != 0) or operands off a
+// fp32 X and W (F32): v_mfma_f32_32x32x2_f32, a sixteenth of the rate, so the
+// matrix cores bound it and 64x64 quadrants are large enough (two workgroups a
+// CU; four sums per output). Against the register-staged 16x16x4 tiles with a
+// K split that these sizes took: [512, 768], N 3072 47.6 -> 32.6 us, 1024 rows
+// 78 -> 51 (94 of the 153 TFLOP/s a large product reaches); [600, 2048], N 2048
+// 107 -> 54; [900, 767], N 3073 124 -> 48; [100, 1147], N 3000 31 -> 16.
+//
+// Rows that are not whole 16-byte chunks (K % 8 != 0, fp32 K % 4) or operands off a
 // 16-byte boundary take the same kernel with the chunks loaded into registers
 // (unaligned 16-byte loads, the last chunk of a row element by element) and
 // written to LDS from there.
@@ -52,16 +59,19 @@ namespace ks {
 // the weight is gemm_pack_weight's copy, whose 16-byte pieces (8 k of one row,
 // 32 rows of a block after each other) are staged in that order: whole
 // contiguous copies, and fragment reads of 1 KB without a swizzle.
-template <int BM_, int BN_, int NW_, int BK_, int S_, bool KSP_, typename TA_, bool DMA_, bool PK_>
+template <int BM_, int BN_, int NW_, int BK_, int S_, bool KSP_, typename TA_, bool DMA_, bool PK_, typename TB_ = half_t>
 struct Cfg {
     static constexpr int BM = BM_, BN = BN_, NW = NW_, BK = BK_, S = DMA_ ? S_ : (KSP_ ? 1 : 2);
     static constexpr bool KSP = KSP_, DMA = DMA_, PK = PK_;
     typedef TA_ TA;
     static constexpr int WM = KSP ? BM : BM / 2, WN = KSP ? BN : BN / 2;   // a wave's part of the tile
+    typedef TB_ TB;
+    static constexpr bool F32 = sizeof(TB_) == 4;              // fp32 W (and X): v_mfma_f32_32x32x2_f32, 8 k a step
+    static constexpr int KQ = F32 ? 8 : 16, KSTEPS = BK / KQ;
     // sums per output and wave (k steps in turn)
-    static constexpr int AS = !KSP ? 1 : WM * WN <= 32 * 64 ? (BK / 16 < 4 || NW == 8 ? 2 : 4) : 2;
-    static constexpr int AES = DMA ? (int)sizeof(TA) : 2;      // X element bytes in LDS
-    static constexpr int AROW = BK * AES, BROW = BK * 2;       // row bytes in LDS
+    static constexpr int AS = F32 ? (KSP ? 2 : 4) : !KSP ? 1 : WM * WN <= 32 * 64 ? (BK / 16 < 4 || NW == 8 ? 2 : 4) : 2;
+    static constexpr int AES = DMA || F32 ? (int)sizeof(TA) : 2, BES = (int)sizeof(TB);   // element bytes in LDS
+    static constexpr int AROW = BK * AES, BROW = BK * BES;       // row bytes in LDS
     static constexpr int ABYTES = BM * AROW, BBYTES = BN * BROW, STAGE = ABYTES + BBYTES;
     static constexpr int SHARE = KSP ? 1 : NW;                 // waves that fill a stage together
     static constexpr int ACOPIES = ABYTES / 1024 / SHARE, BCOPIES = BBYTES / 1024 / SHARE, COPIES = ACOPIES + BCOPIES;
@@ -101,10 +111,12 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 {
     using namespace ks;
     constexpr int BM = C::BM, BN = C::BN, NW = C::NW, BK = C::BK, S = C::S;
-    constexpr int FM = C::WM / 32, FN = C::WN / 32, KSTEPS = BK / 16;
+    constexpr int FM = C::WM / 32, FN = C::WN / 32, KSTEPS = C::KSTEPS;
+    typedef std::conditional_t<C::F32, float4v, half8> frag;   // 16 bytes of one row
     constexpr int BNO = GATED ? BN / 2 : BN;    // output columns per tile
     constexpr int TH = 64 * NW;
     typedef typename C::TA TA;
+    typedef typename C::TB TB;
     extern __shared__ half8 ks_lds[];
     LDS_AS char* lds = (LDS_AS char*)(LDS_AS void*)ks_lds;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -118,7 +130,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     // what every XCD's L2 reads whole.
     const uint32_t w = blockIdx.x, x = w % 8, q8 = tiles / 8, r8 = tiles % 8;
     const uint32_t t = x * q8 + (x < r8 ? x : r8) + w / 8;
-    const bool nmaj = (uint64_t)NO * (GATED ? 4 : 2) >= (uint64_t)M * sizeof(TA);
+    const bool nmaj = (uint64_t)NO * (GATED ? 2 : 1) * sizeof(TB) >= (uint64_t)M * sizeof(TA);
     const uint32_t tm = __builtin_amdgcn_readfirstlane(nmaj ? t % tiles_m : t / tiles_n);
     const uint32_t tn = __builtin_amdgcn_readfirstlane(nmaj ? t / tiles_m : t % tiles_n);
     const uint32_t m0 = tm * BM, n0 = tn * BNO;
@@ -128,7 +140,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     const int wm0 = C::KSP ? 0 : (wave >> 1) * C::WM, wn0 = C::KSP ? 0 : (wave & 1) * C::WN;
 
     const TA* A = (const TA*)p.A;
-    const half_t* B = (const half_t*)p.B;
+    const TB* B = (const TB*)p.B;
     // W row of the tile's logical column j (clamped into W; a column past the
     // output is never stored)
     const auto wrow = [&](uint32_t j) __attribute__((always_inline)) {
@@ -148,10 +160,10 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     // s % CH. Rows past M read as zero (out of the resource's range), chunks
     // past the row's end too (an offset past any range).
     constexpr int ACH = C::AROW / 16, BCH = C::BROW / 16;
-    constexpr int AEC = 16 / C::AES;            // X elements per chunk
+    constexpr int AEC = 16 / C::AES, BEC = 16 / C::BES;   // elements per chunk
     uint32_t aoff[C::ACOPIES], boff[C::BCOPIES];
     __amdgpu_buffer_rsrc_t ra, rb;
-    half8 sa[C::DMA ? 1 : C::ACOPIES], sb[C::DMA ? 1 : C::BCOPIES];
+    frag sa[C::DMA ? 1 : C::ACOPIES], sb[C::DMA ? 1 : C::BCOPIES];
     if constexpr (C::DMA) {
         ra = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(A + (size_t)m0 * K), (short)0,
                                                (int)__builtin_amdgcn_readfirstlane((M - m0) * K * (uint32_t)sizeof(TA)),
@@ -165,7 +177,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
                                                    0x00020000);
         else
             rb = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(B), (short)0,
-                                                   (int)__builtin_amdgcn_readfirstlane((GATED ? 2 * H : N) * K * 2), 0x00020000);
+                                                   (int)__builtin_amdgcn_readfirstlane((GATED ? 2 * H : N) * K * (uint32_t)sizeof(TB)), 0x00020000);
 #pragma unroll
         for (int i = 0; i < C::ACOPIES; ++i) {
             const int s = (cw * C::ACOPIES + i) * 64 + lane, row = s / ACH, ch = swz<C::AROW>(row, s % ACH);
@@ -182,7 +194,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
                 boff[i] = blk * K * 64 + (ch * 32 + jo % 32) * 16;
             } else {
                 const int row = s / BCH, ch = swz<C::BROW>(row, s % BCH);
-                boff[i] = (wrow(row) * K + ch * 8) * 2;
+                boff[i] = (wrow(row) * K + ch * BEC) * (uint32_t)sizeof(TB);
             }
         }
     }
@@ -206,8 +218,8 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
         for (int i = C::BCOPIES * q / KSTEPS; i < C::BCOPIES * (q + 1) / KSTEPS; ++i) {
             const int s = (cw * C::BCOPIES + i) * 64 + lane, ch = C::PK ? s / BN : swz<C::BROW>(s / BCH, s % BCH);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_AS void*)(bdst + i * 1024), 16,
-                                                     (int)((uint32_t)ch * 8 < left ? boff[i] : 0x80000000u),
-                                                     (int)(k0 * (C::PK ? 64 : 2)), 0, 0);
+                                                     (int)((uint32_t)ch * BEC < left ? boff[i] : 0x80000000u),
+                                                     (int)(k0 * (C::PK ? 64 : (int)sizeof(TB))), 0, 0);
         }
     };
     const auto issue = [&](int slot, int c) __attribute__((always_inline)) {
@@ -216,32 +228,35 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     };
     // Register staging of chunk c, and its write into a stage. Rows past M
     // read row M - 1 (their outputs are never stored); a piece past the row's
-    // last 8 elements reads those and moves them down.
+    // last PE elements reads those and moves them down.
+    constexpr int PE = C::F32 ? 4 : 8;          // elements per piece
     const auto fetch = [&](int c) __attribute__((always_inline)) {
         const uint32_t k0 = (uint32_t)c * BK;
         const bool whole = k0 + BK <= K;
+        const auto piece = [&](const auto* row, uint32_t k) __attribute__((always_inline)) {
+            if constexpr (C::F32) return load4f(row + std::min(k, K - PE));
+            else return load8(row + std::min(k, K - PE));
+        };
 #pragma unroll
         for (int i = 0; i < C::ACOPIES; ++i) {
             const int s = (cw * C::ACOPIES + i) * 64 + lane;
-            const uint32_t k = k0 + (s % ACH) * 8, m = std::min(m0 + s / ACH, M - 1);
-            sa[i] = load8(A + (size_t)m * K + std::min(k, K - 8));
+            sa[i] = piece(A + (size_t)std::min(m0 + s / ACH, M - 1) * K, k0 + (s % ACH) * PE);
         }
 #pragma unroll
         for (int i = 0; i < C::BCOPIES; ++i) {
             const int s = (cw * C::BCOPIES + i) * 64 + lane;
-            const uint32_t k = k0 + (s % BCH) * 8;
-            sb[i] = load8(B + (size_t)wrow(s / BCH) * K + std::min(k, K - 8));
+            sb[i] = piece(B + (size_t)wrow(s / BCH) * K, k0 + (s % BCH) * PE);
         }
         if (!whole) {
 #pragma unroll
             for (int i = 0; i < C::ACOPIES; ++i) {
-                const uint32_t k = k0 + (((cw * C::ACOPIES + i) * 64 + lane) % ACH) * 8;
-                sa[i] = shift_down(sa[i], std::min(k - std::min(k, K - 8), 8u));
+                const uint32_t k = k0 + (((cw * C::ACOPIES + i) * 64 + lane) % ACH) * PE;
+                sa[i] = shift_down(sa[i], std::min<uint32_t>(k - std::min(k, K - PE), PE));
             }
 #pragma unroll
             for (int i = 0; i < C::BCOPIES; ++i) {
-                const uint32_t k = k0 + (((cw * C::BCOPIES + i) * 64 + lane) % BCH) * 8;
-                sb[i] = shift_down(sb[i], std::min(k - std::min(k, K - 8), 8u));
+                const uint32_t k = k0 + (((cw * C::BCOPIES + i) * 64 + lane) % BCH) * PE;
+                sb[i] = shift_down(sb[i], std::min<uint32_t>(k - std::min(k, K - PE), PE));
             }
         }
     };
@@ -250,20 +265,21 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
         for (int i = 0; i < C::ACOPIES; ++i) {
             const int s = (cw * C::ACOPIES + i) * 64 + lane, row = s / ACH;
-            *(LDS_AS half8*)(st + row * C::AROW + swz<C::AROW>(row, s % ACH) * 16) = sa[i];
+            *(LDS_AS frag*)(st + row * C::AROW + swz<C::AROW>(row, s % ACH) * 16) = sa[i];
         }
 #pragma unroll
         for (int i = 0; i < C::BCOPIES; ++i) {
             const int s = (cw * C::BCOPIES + i) * 64 + lane, row = s / BCH;
-            *(LDS_AS half8*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, s % BCH) * 16) = sb[i];
+            *(LDS_AS frag*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, s % BCH) * 16) = sb[i];
         }
     };
 
-    // ---- fragments: row i*32 + fr of the wave's part, 16-wide k step q ----
+    // ---- fragments: row i*32 + fr of the wave's part, k step q (lane half fk:
+    // 8 of its 16, or 4 of its 8 fp32) ----
     const auto read_x = [&](const LDS_AS char* st, int i, int q) __attribute__((always_inline)) {
         const int row = wm0 + i * 32 + fr;
-        if constexpr (C::AES == 2) {
-            return *(const LDS_AS half8*)(st + row * C::AROW + swz<C::AROW>(row, q * 2 + fk) * 16);
+        if constexpr (C::AES == 2 || C::F32) {
+            return *(const LDS_AS frag*)(st + row * C::AROW + swz<C::AROW>(row, q * 2 + fk) * 16);
         } else {
             const float4v lo = *(const LDS_AS float4v*)(st + row * C::AROW + swz<C::AROW>(row, q * 4 + 2 * fk) * 16);
             const float4v hi = *(const LDS_AS float4v*)(st + row * C::AROW + swz<C::AROW>(row, q * 4 + 2 * fk + 1) * 16);
@@ -274,7 +290,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     const auto read_w = [&](const LDS_AS char* st, int j, int q) __attribute__((always_inline)) {
         const int row = wn0 + j * 32 + fr;
         if constexpr (C::PK) return *(const LDS_AS half8*)(st + C::ABYTES + ((q * 2 + fk) * BN + row) * 16);
-        return *(const LDS_AS half8*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, q * 2 + fk) * 16);
+        else return *(const LDS_AS frag*)(st + C::ABYTES + row * C::BROW + swz<C::BROW>(row, q * 2 + fk) * 16);
     };
 
     // This thread's output columns in the final exchange (the same for each of
@@ -310,7 +326,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     // MFMAs), the shared ring's waves read one step ahead.
     const auto stage_mfma = [&](const LDS_AS char* st, auto&& step) __attribute__((always_inline)) {
         constexpr int AHEAD = C::KSP ? KSTEPS : 1, SETS = C::KSP ? KSTEPS : 2;
-        half8 xf[SETS][FM], wf[SETS][FN];
+        frag xf[SETS][FM], wf[SETS][FN];
 #pragma unroll
         for (int q = 0; q < AHEAD; ++q) {
 #pragma unroll
@@ -327,12 +343,24 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
                 for (int j = 0; j < FN; ++j) wf[(q + AHEAD) % SETS][j] = read_w(st, j, q + AHEAD);
             }
+            if constexpr (C::F32) {
+                // element e of both halves' pieces is one k pair (the same on both operands)
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[q % AS][i][j] =
-                        __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[q % SETS][j], xf[q % SETS][i], acc[q % AS][i][j], 0, 0, 0);
+                    for (int i = 0; i < FM; ++i)
+#pragma unroll
+                        for (int j = 0; j < FN; ++j)
+                            acc[e % AS][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                wf[q % SETS][j][e], xf[q % SETS][i][e], acc[e % AS][i][j], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[q % AS][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[q % SETS][j], xf[q % SETS][i],
+                                                                                   acc[q % AS][i][j], 0, 0, 0);
+            }
             if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
             step(q);
             if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
@@ -527,33 +555,36 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     }
 }
 
-// fp16 W, fp16 or fp32 X, 32-bit buffer offsets.
+// fp16 W with fp16 or fp32 X, or both fp32 (ungated); 32-bit buffer offsets.
 bool gemm_ksplit_ok(const GemmParams& p, bool gated)
 {
-    const uint64_t as = p.a_dtype == DT_F16 ? 2 : 4;
-    return p.b_dtype == DT_F16 && p.batch == 1 && (uint64_t)p.M * p.K * as < (1ull << 31) &&
-           (uint64_t)p.N * p.K * 2 < (1ull << 31) && (uint64_t)p.M * p.N < (1ull << 31) && p.K >= 32 && p.K < (1u << 22) &&
-           (!gated || p.H > 0);
+    const uint64_t as = p.a_dtype == DT_F16 ? 2 : 4, bs = p.b_dtype == DT_F16 ? 2 : 4;
+    return (p.b_dtype == DT_F16 || (p.a_dtype == DT_F32 && !gated)) && p.batch == 1 &&
+           (uint64_t)p.M * p.K * as < (1ull << 31) && (uint64_t)p.N * p.K * bs < (1ull << 31) &&
+           (uint64_t)p.M * p.N < (1ull << 31) && p.K >= 32 && p.K < (1u << 22) && (!gated || p.H > 0);
 }
 
 // The tiles offered. A launch takes about 2.5 us plus, per round of tiles over
-// the CUs, `fixed` plus `chunk` per 64 k (us; index 0: fp16 X, 1: fp32 X;
-// measured on full grids at K = 768 and 2048).
+// the CUs, `fixed` plus `chunk` per 64 k (us; index 0: fp16 X, 1: fp32 X, 2:
+// fp32 X and W; measured on full grids at K = 768 and 2048). fp32 products run
+// at 1/16 of the fp16 rate: operands take a quarter of the time and only the
+// smallest quadrants and K-split tiles are of use.
 namespace ks {
-struct Tile { int bm, bn; float fixed[2], chunk[2]; };
+struct Tile { int bm, bn; float fixed[3], chunk[3]; };
+constexpr float NONE = 1e9f;
 constexpr Tile TILES[] = {
-    {32, 32, {2.2f, 1.7f}, {.091f, .165f}},     // 8 waves split K
-    {32, 64, {2.2f, 2.3f}, {.14f, .18f}},       // 4 waves split K
-    {64, 64, {2.85f, 1.7f}, {.17f, .37f}},
-    {64, 128, {2.3f, 2.7f}, {.39f, .465f}},     // quadrants
-    {128, 128, {4.0f, 2.3f}, {.55f, .84f}},
+    {32, 32, {2.2f, 1.7f, 1.5f}, {.091f, .165f, .31f}},     // 8 waves split K
+    {32, 64, {2.2f, 2.3f, NONE}, {.14f, .18f, 0.f}},        // 4 waves split K
+    {64, 64, {2.85f, 1.7f, 2.3f}, {.17f, .37f, 1.1f}},      // (fp32: quadrants)
+    {64, 128, {2.3f, 2.7f, NONE}, {.39f, .465f, 0.f}},      // quadrants
+    {128, 128, {4.0f, 2.3f, NONE}, {.55f, .84f, 0.f}},
 };
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 
 // Whole 16-byte chunks everywhere: the copies go straight to LDS.
 inline bool dma_ok(const GemmParams& p)
 {
-    return p.K % 8 == 0 && ((uintptr_t)p.A % 16) == 0 && ((uintptr_t)p.B % 16) == 0;
+    return p.K % (p.b_dtype == DT_F16 ? 8 : 4) == 0 && ((uintptr_t)p.A % 16) == 0 && ((uintptr_t)p.B % 16) == 0;
 }
 }
 
@@ -565,15 +596,18 @@ void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn)
 
 int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
 {
-    const int x = p.a_dtype == DT_F16 ? 0 : 1;
-    const float chunks = (float)((p.K + 63) / 64) * (ks::dma_ok(p) ? 1.f : 1.7f);   // (register staging: 1.5-1.9)
+    const int x = p.b_dtype == DT_F32 ? 2 : p.a_dtype == DT_F16 ? 0 : 1;
+    // (register staging: fp16 1.5-1.9; fp32 measured alike, 15.2 us a tile at K = 767 and 768)
+    const float chunks = (float)((p.K + 63) / 64) * (ks::dma_ok(p) || x == 2 ? 1.f : 1.7f);
     const uint32_t cols = gated ? 2 * p.H : p.N;
     int best = 0;
     *us = 1e30f;
     for (int t = 0; t < ks::NTILES; ++t) {
         const ks::Tile& k = ks::TILES[t];
         const uint64_t tiles = (uint64_t)((p.M + k.bm - 1) / k.bm) * ((cols + k.bn - 1) / k.bn);
-        const float cost = 2.5f + (float)((tiles + cus - 1) / cus) * (k.fixed[x] + chunks * k.chunk[x]);
+        // (fp32 quadrants alone on a CU, one wave per SIMD: 22 us where a pair takes 2 x 19)
+        const float rounds = (float)((tiles + cus - 1) / cus) * (x == 2 && k.bm == 64 && tiles <= cus ? 1.15f : 1.f);
+        const float cost = 2.5f + rounds * (k.fixed[x] + chunks * k.chunk[x]);
         if (cost < *us) { *us = cost; best = t; }
     }
     return best;
@@ -611,9 +645,17 @@ static hipError_t launch_gate(const GemmParams& p, const void* packed, bool gate
     return gated ? launch_tile<TA, DMA, PK, true>(p, packed, tile, s) : launch_tile<TA, DMA, PK, false>(p, packed, tile, s);
 }
 
+template <bool DMA>
+static hipError_t launch_f32(const GemmParams& p, int tile, hipStream_t s)
+{
+    if (tile == 0) return launch_cfg<ks::Cfg<32, 32, 8, 32, 2, true, float, DMA, false, float>, false>(p, nullptr, s);
+    return launch_cfg<ks::Cfg<64, 64, 4, 32, 4, false, float, DMA, false, float>, false>(p, nullptr, s);
+}
+
 hipError_t gemm_ksplit_launch(const GemmParams& p, const void* packed, bool gated, int tile, hipStream_t s)
 {
     const bool dma = ks::dma_ok(p);
+    if (p.b_dtype == DT_F32) return dma ? launch_f32<true>(p, tile, s) : launch_f32<false>(p, tile, s);
     if (p.a_dtype == DT_F16) {
         // (the packed form has K % 128 == 0: no short chunk). The weight itself
         // is then not read, as in the 256x256 kernel over the packed form.
