@@ -291,7 +291,89 @@ __global__ __launch_bounds__(256) void slab_vec_kernel(SlabParams a)
     store_output(slab_output(a), (size_t)m * N + n0 + r, acc[0]);
 }
 
-// Any K, any alignment: one wave per output column, scalar loads.
+// Any K from one chunk up, elements at any address: rows that are not whole
+// 16-byte chunks, or operands off a 16-byte boundary. A wave owns R rows and
+// takes chunks of EPC elements by unaligned 16-byte loads (one element a load,
+// 2 bytes a lane, was bound by the number of loads: M = 8, K = 1148, N = 22480
+// 130 us, now 16; M = 1, K = 2047, N = 8192 21 us, now 7). The row's last,
+// short chunk reads its last EPC elements and drops those already taken, in W
+// and in X (a dropped infinity must not meet a zero).
+template <int MP, int R, typename TI, typename TW>
+__global__ __launch_bounds__(256) void slab_any_kernel(SlabParams a)
+{
+    constexpr int EPC = Vec16<TW>::n, V = MP * R, KCH = MP == 8 ? 1 : 2;
+    static_assert(V <= 64 && (V & (V - 1)) == 0, "butterfly needs a power of two <= 64");
+    typedef TW wvec __attribute__((ext_vector_type(EPC)));
+    typedef TI xvec __attribute__((ext_vector_type(EPC)));
+    typedef wvec wvecu __attribute__((aligned(sizeof(TW))));
+    typedef xvec xvecu __attribute__((aligned(sizeof(TI))));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n0 = (blockIdx.x * 4u + wave) * R;
+    const uint32_t K = a.K, N = a.N, M = a.M;
+    if (n0 >= N) return;
+    // rows past N and M read the last row and row 0: never stored
+    const TW* w[R];
+    const TI* x[MP];
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = (const TW*)a.weight + (size_t)std::min(n0 + r, N - 1) * K;
+#pragma unroll
+    for (int m = 0; m < MP; ++m) x[m] = (const TI*)a.in + (size_t)((uint32_t)m < M ? m : 0) * K;
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+
+    const auto block = [&](uint32_t kb, auto whole_c, auto chunks_c) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(whole_c)::value;
+        constexpr int C = decltype(chunks_c)::value;
+        wvec wv[C][R];
+        xvec xv[C][MP];
+        uint32_t drop[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const uint32_t k = kb + (uint32_t)(c * 64 + lane) * EPC, kc = WHOLE ? k : std::min(k, K - EPC);
+            drop[c] = std::min<uint32_t>(k - kc, EPC);
+#pragma unroll
+            for (int r = 0; r < R; ++r) wv[c][r] = *(const wvecu*)(w[r] + kc);
+#pragma unroll
+            for (int m = 0; m < MP; ++m) xv[c][m] = *(const xvecu*)(x[m] + kc);
+        }
+        if constexpr (!WHOLE) {
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int e = 0; e < EPC; ++e) {
+                    const bool out = (uint32_t)e < drop[c];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) wv[c][r][e] = out ? (TW)0 : wv[c][r][e];
+#pragma unroll
+                    for (int m = 0; m < MP; ++m) xv[c][m][e] = out ? (TI)0 : xv[c][m][e];
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int m = 0; m < MP; ++m)
+#pragma unroll
+                for (int r = 0; r < R; ++r) acc[m * R + r] = chunk_dot<TI, TW>(wv[c][r], xv[c][m], acc[m * R + r]);
+    };
+    uint32_t kb = 0;
+    for (; kb + 64 * EPC * KCH <= K; kb += 64 * EPC * KCH) block(kb, std::true_type{}, std::integral_constant<int, KCH>{});
+    for (; kb < K; kb += 64 * EPC) {
+        if (kb + 64 * EPC <= K) block(kb, std::true_type{}, std::integral_constant<int, 1>{});
+        else block(kb, std::false_type{}, std::integral_constant<int, 1>{});
+    }
+
+    butterfly<V, 32>(acc, lane);
+    const int idx = butterfly_index<V>(lane);
+    if ((lane & (butterfly_low<V>() - 1)) != 0) return;
+    const uint32_t m = idx / R, r = idx % R;
+    if (m >= M || n0 + r >= N) return;
+    store_output(slab_output(a), (size_t)m * N + n0 + r, acc[0]);
+}
+
+// K shorter than one chunk, or elements off their own alignment: one wave per
+// output column, one element a lane.
 template <int MP>
 __global__ __launch_bounds__(256) void slab_scalar_kernel(SlabParams a)
 {
@@ -415,6 +497,21 @@ static hipError_t launch_m(const SlabParams& a, hipStream_t s)
     return launch_vec<MP, float, float>(a, s);
 }
 
+template <int MP>
+static hipError_t launch_any(const SlabParams& a, hipStream_t s)
+{
+    constexpr int R = MP == 8 ? 4 : 2;
+    const dim3 grid((a.N + 4 * R - 1) / (4 * R)), block(256);
+    if (a.w_dtype == DT_F16) {
+        if (a.i_dtype == DT_F16) hipLaunchKernelGGL((slab_any_kernel<MP, R, half_t, half_t>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((slab_any_kernel<MP, R, float, half_t>), grid, block, 0, s, a);
+    } else if (a.i_dtype == DT_F16)
+        hipLaunchKernelGGL((slab_any_kernel<MP, R, half_t, float>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((slab_any_kernel<MP, R, float, float>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
 bool slab_vec_ok(const SlabParams& a)
 {
     const uint32_t epc = a.w_dtype == DT_F16 ? 8 : 4;
@@ -439,6 +536,15 @@ hipError_t slab_launch(const SlabParams& a, hipStream_t s)
         case 2: return launch_m<2>(a, s);
         case 3: case 4: return launch_m<4>(a, s);
         default: return launch_m<8>(a, s);
+        }
+    }
+    const uintptr_t is = a.i_dtype == DT_F16 ? 2 : 4, wsz = a.w_dtype == DT_F16 ? 2 : 4;
+    if (a.K >= 8 && (uintptr_t)a.in % is == 0 && (uintptr_t)a.weight % wsz == 0) {
+        switch (a.M) {
+        case 1: return launch_any<1>(a, s);
+        case 2: return launch_any<2>(a, s);
+        case 3: case 4: return launch_any<4>(a, s);
+        default: return launch_any<8>(a, s);
         }
     }
     const uint32_t blocks = (a.N + 3) / 4;
