@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 F16, F32 = np.float16, np.float32
 
 
-def run(gpu, x, w, odt, xoff=0, woff=0):
+def run(gpu, x, w, odt, xoff=0, woff=0, plan="slab_scalar"):
     D = gpu.DeviceArray.from_numpy
     dx = D(np.concatenate([np.full(xoff, np.nan, x.dtype), x.ravel(), np.full(9, np.nan, x.dtype)]))
     dw = D(np.concatenate([np.full(woff, np.nan, w.dtype), w.ravel(), np.full(9, np.nan, w.dtype)]))
@@ -22,7 +22,7 @@ def run(gpu, x, w, odt, xoff=0, woff=0):
     a.inp, a.weight = dx.ptr + x.itemsize * xoff, dw.ptr + w.itemsize * woff
     name = gpu.linear_plan(a)[0]
     print(f"slab m={x.shape[0]} k={x.shape[1]} n={w.shape[0]} {x.dtype} x {w.dtype} -> {name}", flush=True)
-    assert name == "slab_scalar"
+    assert name == plan
     gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
     gpu.synchronize()
     return out.numpy().astype(np.float64)
@@ -43,14 +43,28 @@ def run(gpu, x, w, odt, xoff=0, woff=0):
     (8, 512, 40, F32, F16, F32, (1, 0)),         # X off a boundary
     (6, 260, 21, F32, F32, F32, (3, 2)),
 ])
-def test_slab_any(gpu, m, k, n, xdt, wdt, odt, off):
+def test_slab_any(gpu, m, k, n, xdt, wdt, odt, off, plan="slab_scalar"):
     rng = np.random.default_rng(m + k + n)
     x, w = draw((m, k), rng, xdt), draw(normal((n, k), 0.1), rng, wdt)
-    got = run(gpu, x, w, odt, *off)
+    got = run(gpu, x, w, odt, *off, plan=plan)
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     y = x64 @ w64.T
     tol = (np.abs(x64) @ np.abs(w64).T) * (k + 1) * 2.0 ** -24 + (2.0 ** -11 * np.abs(y) + 2.0 ** -24 if odt == F16 else 1e-30)
     assert np.isfinite(got).all() and (np.abs(got - y) <= tol).all(), float((np.abs(got - y) / tol).max())
+
+
+@pytest.mark.parametrize("m, k, n, xdt, wdt, odt", [
+    (8, 1000, 1023, F16, F16, F32),       # one row a wave
+    (5, 520, 1024, F32, F16, F32),        # two
+    (8, 1000, 2050, F16, F16, F16),       # four, the last wave's partly past N
+    (8, 1024, 2047, F32, F32, F32),       # fp32 rows: two a wave ...
+    (6, 1028, 2049, F32, F32, F32),       # ... and X through LDS
+    (4, 1032, 1030, F32, F16, F32),
+    (3, 516, 17, F32, F32, F32),
+])
+def test_slab_whole_chunks(gpu, m, k, n, xdt, wdt, odt):
+    """Rows of whole chunks with more activations than a lane holds ahead."""
+    test_slab_any(gpu, m, k, n, xdt, wdt, odt, (0, 0), plan="slab")
 
 
 def test_slab_any_infinity(gpu):

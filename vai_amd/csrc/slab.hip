@@ -216,8 +216,11 @@ __global__ __launch_bounds__(256) void slab_reg_kernel(const TW* __restrict__ Wp
 }
 
 
-// More input rows (5-8, or 3-8 with fp32 input): the M rows of each K block
-// are staged once per workgroup in LDS and broadcast to the four waves.
+// 5-8 input rows against many long fp32 rows: the M rows of each K block are
+// staged once per workgroup in LDS and broadcast to the four waves (the X of
+// each wave would be twice its W bytes: K = 2048, N = 4096 11.3 us, 11.6-12.7
+// without; below, the barriers cost more: K = 768, N = 3072 5.7 against 4.8,
+// K = 3072, N = 768 11.0 against 7.2).
 template <int MP, int R, int KCH, typename TI, typename TW>
 __global__ __launch_bounds__(256) void slab_vec_kernel(SlabParams a)
 {
@@ -301,7 +304,7 @@ __global__ __launch_bounds__(256) void slab_vec_kernel(SlabParams a)
 template <int MP, int R, typename TI, typename TW>
 __global__ __launch_bounds__(256) void slab_any_kernel(SlabParams a)
 {
-    constexpr int EPC = Vec16<TW>::n, V = MP * R, KCH = MP == 8 ? 1 : 2;
+    constexpr int EPC = Vec16<TW>::n, V = MP * R, KCH = R == 4 ? 1 : 2;
     static_assert(V <= 64 && (V & (V - 1)) == 0, "butterfly needs a power of two <= 64");
     typedef TW wvec __attribute__((ext_vector_type(EPC)));
     typedef TI xvec __attribute__((ext_vector_type(EPC)));
@@ -467,6 +470,22 @@ bool gemv_mfma_ok(const SlabParams& a)
            ((uintptr_t)a.weight % 16) == 0 && ((uintptr_t)a.in % 16) == 0;
 }
 
+// R rows a wave (each X chunk then serves R rows) where that leaves 128
+// workgroups: M = 8, K = 8192, N = 2048 in 128 workgroups of R = 4 18.3 us, in
+// 512 of R = 1 20.5; K = 3072, N = 768 in 48 9.5 (fp32 12.2), in 192 5.3 (7.3).
+template <int MP, typename TI, typename TW>
+static hipError_t launch_any(const SlabParams& a, hipStream_t s)
+{
+    constexpr int RMAX = MP == 8 ? 4 : 2;
+    const auto go = [&](auto R) {
+        hipLaunchKernelGGL((slab_any_kernel<MP, R, TI, TW>), dim3((a.N + 4 * R - 1) / (4 * R)), dim3(256), 0, s, a);
+        return hipGetLastError();
+    };
+    if (a.N >= 4 * RMAX * 128) return go(std::integral_constant<int, RMAX>{});
+    if (RMAX > 2 && a.N >= 4 * 2 * 128) return go(std::integral_constant<int, 2>{});
+    return go(std::integral_constant<int, 1>{});
+}
+
 template <int MP, typename TI, typename TW>
 static hipError_t launch_vec(const SlabParams& a, hipStream_t s)
 {
@@ -483,33 +502,33 @@ static hipError_t launch_vec(const SlabParams& a, hipStream_t s)
         else
             hipLaunchKernelGGL((slab_reg_kernel<MP, R, KCH, TI, TW, false>), dim3(blocks), dim3(256), 0, s,
                                (const TW*)a.weight, (const TI*)a.in, a.K, a.N, a.M, a);
-    } else
-        hipLaunchKernelGGL((slab_vec_kernel<MP, R, KCH, TI, TW>), dim3(blocks), dim3(256), 0, s, a);
-    return hipGetLastError();
+        return hipGetLastError();
+    } else {
+        if constexpr (MP == 8 && sizeof(TW) == 4)
+            if (a.N >= 2048 && a.K >= 1024) {
+                hipLaunchKernelGGL((slab_vec_kernel<MP, R, KCH, TI, TW>), dim3(blocks), dim3(256), 0, s, a);
+                return hipGetLastError();
+            }
+        // more rows than a lane's registers hold in four chunks: R rows a wave,
+        // X from L2 (against the rows staged in LDS: fp16 W, M = 8, K = 2048,
+        // N = 8192 15.4 -> 13.3 us; K = 3072, N = 768 9.8 -> 5.3; fp16 X,
+        // K = 1000, N = 3000 6.7 -> 4.2)
+        return launch_any<MP, TI, TW>(a, s);
+    }
 }
 
 template <int MP>
-static hipError_t launch_m(const SlabParams& a, hipStream_t s)
+static hipError_t launch_m(const SlabParams& a, bool vec, hipStream_t s)
 {
-    if (a.i_dtype == DT_F16 && a.w_dtype == DT_F16) return launch_vec<MP, half_t, half_t>(a, s);
-    if (a.i_dtype == DT_F32 && a.w_dtype == DT_F16) return launch_vec<MP, float, half_t>(a, s);
-    if (a.i_dtype == DT_F16 && a.w_dtype == DT_F32) return launch_vec<MP, half_t, float>(a, s);
-    return launch_vec<MP, float, float>(a, s);
-}
-
-template <int MP>
-static hipError_t launch_any(const SlabParams& a, hipStream_t s)
-{
-    constexpr int R = MP == 8 ? 4 : 2;
-    const dim3 grid((a.N + 4 * R - 1) / (4 * R)), block(256);
-    if (a.w_dtype == DT_F16) {
-        if (a.i_dtype == DT_F16) hipLaunchKernelGGL((slab_any_kernel<MP, R, half_t, half_t>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((slab_any_kernel<MP, R, float, half_t>), grid, block, 0, s, a);
-    } else if (a.i_dtype == DT_F16)
-        hipLaunchKernelGGL((slab_any_kernel<MP, R, half_t, float>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((slab_any_kernel<MP, R, float, float>), grid, block, 0, s, a);
-    return hipGetLastError();
+    const auto go = [&](auto ti, auto tw) {
+        typedef decltype(ti) TI;
+        typedef decltype(tw) TW;
+        return vec ? launch_vec<MP, TI, TW>(a, s) : launch_any<MP, TI, TW>(a, s);
+    };
+    if (a.i_dtype == DT_F16 && a.w_dtype == DT_F16) return go(half_t{}, half_t{});
+    if (a.i_dtype == DT_F32 && a.w_dtype == DT_F16) return go(float{}, half_t{});
+    if (a.i_dtype == DT_F16 && a.w_dtype == DT_F32) return go(half_t{}, float{});
+    return go(float{}, float{});
 }
 
 bool slab_vec_ok(const SlabParams& a)
@@ -530,21 +549,14 @@ hipError_t slab_launch(const SlabParams& a, hipStream_t s)
         hipLaunchKernelGGL(gemv_lds_kernel, dim3((a.N + 15) / 16), dim3(256), 65536, s, a);
         return hipGetLastError();
     }
-    if (slab_vec_ok(a)) {
+    const uintptr_t isz = a.i_dtype == DT_F16 ? 2 : 4, wsz = a.w_dtype == DT_F16 ? 2 : 4;
+    const bool vec = slab_vec_ok(a);
+    if (vec || (a.K >= 8 && (uintptr_t)a.in % isz == 0 && (uintptr_t)a.weight % wsz == 0)) {
         switch (a.M) {
-        case 1: return launch_m<1>(a, s);
-        case 2: return launch_m<2>(a, s);
-        case 3: case 4: return launch_m<4>(a, s);
-        default: return launch_m<8>(a, s);
-        }
-    }
-    const uintptr_t is = a.i_dtype == DT_F16 ? 2 : 4, wsz = a.w_dtype == DT_F16 ? 2 : 4;
-    if (a.K >= 8 && (uintptr_t)a.in % is == 0 && (uintptr_t)a.weight % wsz == 0) {
-        switch (a.M) {
-        case 1: return launch_any<1>(a, s);
-        case 2: return launch_any<2>(a, s);
-        case 3: case 4: return launch_any<4>(a, s);
-        default: return launch_any<8>(a, s);
+        case 1: return launch_m<1>(a, vec, s);
+        case 2: return launch_m<2>(a, vec, s);
+        case 3: case 4: return launch_m<4>(a, vec, s);
+        default: return launch_m<8>(a, vec, s);
         }
     }
     const uint32_t blocks = (a.N + 3) / 4;
