@@ -21,6 +21,9 @@ F16, F32 = np.float16, np.float32
     (1, 72, 24, 520, 520, 80, True, 70, F16),      # window, padded head dim
     (3, 43, 43, 300, 300, 256, True, 0, F32),
     (1, 24, 8, 1000, 1000, 128, True, 0, F32),     # fewer tiles than CUs: split
+    (1, 24, 8, 1400, 1400, 128, True, 0, F32),     # two wave groups share the keys, unsplit, odd and even walks
+    (1, 40, 40, 833, 900, 64, True, 0, F16),
+    (1, 2, 2, 640, 640, 72, False, 0, F32),        # ... and split
     (1, 16, 2, 256, 2111, 128, True, 0, F16),      # long walks, an odd number of tiles
     (1, 4, 4, 64, 65, 64, False, 0, F32),
     (1, 2, 2, 100, 64, 128, False, 0, F16),        # one key tile

@@ -238,17 +238,23 @@ __device__ __forceinline__ void fa_wait_vmcnt()
 // with one wave per SIMD and each head's walks in turn, 122 us now, 840 TFLOP/s
 // of visible work; the LDS fragment reads (128 KB a tile and workgroup) bound it
 // next. D = 256 needs 392 registers and 128 KB: one workgroup per CU.
-template <int D>
-__global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention_fwd_kernel(AttnParams p)
+//
+// KG = 2: where there is only one workgroup for a CU (the grid, or a split's
+// one round), eight waves: two groups of four take the key tiles in turn, each
+// with its own stages, (m, l) and O, and the second hands its to the first
+// through LDS at the end (by register image: the lanes agree).
+template <int D, int KG>
+__global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 : 1) void attention_fwd_kernel(AttnParams p)
 {
     using namespace fa;
     using L = Lds<D>;
     const uint32_t HD = p.head_dim, ROWG = HD * 2;   // head dim and K / V row bytes in HBM
     constexpr int KS = D / 16, DF = D / 32;   // 16-wide head-dim steps; 32-wide output fragments
     extern __shared__ half8 fa_lds[];
-    LDS_AS char* lds = (LDS_AS char*)(LDS_AS void*)fa_lds;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = KG == 1 ? wid : wid & 3, kg = KG == 1 ? 0 : wid >> 2;   // query rows of the tile; key group
+    LDS_AS char* lds = (LDS_AS char*)(LDS_AS void*)fa_lds + kg * L::BYTES;
     const int ql = lane & 31, hf = lane >> 5;   // lane's query (of the wave's 32) and lane half
     const uint32_t Tq = p.tq;
     // keys: positions [0, live); with a cache, its count is read here, at run time
@@ -363,7 +369,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention
         return __builtin_amdgcn_make_buffer_rsrc((void*)(h + (size_t)row0 * ROWG), (short)0, (int)(rows * ROWG),
                                                  0x00020000);
     };
-    if (ntiles > 0) fa_issue<D>(rsrc(0, kh0), rsrc(0, vh0), lds, coff, 0, wave);
+    if (kg < ntiles) fa_issue<D>(rsrc(kg, kh0), rsrc(kg, vh0), lds, coff, 0, wave);
 
     // (the rest of the set-up runs while Q and the first tiles load)
     const float sl2 = p.scale * 1.4426950408889634f;   // scores in log2 units
@@ -394,19 +400,21 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention
         vofs[j] = lds0 + (vkey + vrow) * L::ROWB + ((4 * j + (vcol >> 3)) ^ swz_f((vkey + vrow) & 7)) * 16 +
                   (vcol & 7) * 2;
 
-    for (int t = 0; t < ntiles; ++t) {
-        // Tile t landed in every wave's share: nothing younger is in flight
-        // (tile t + 1's copies are issued during tile t's S^T MFMAs, a few
+    for (int t = 0; KG * t < ntiles; ++t) {
+        // Tile T = kg + KG t of the unit, in stage t % 2 of the group. It landed in every wave's share: nothing younger is in flight
+        // (tile T + KG's copies are issued during tile T's S^T MFMAs, a few
         // per group, so that the wave does not stall on a burst of them).
         fa_wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
+        const int T = kg + KG * t;
+        if (KG == 1 || T < ntiles) {   // (an odd last tile leaves the second group only the barriers)
         const uint32_t sb = (t & 1) * L::STAGE;
         uint32_t kaddr[NK], vaddr[2];
 #pragma unroll
         for (int j = 0; j < NK; ++j) kaddr[j] = kofs[j] + sb;
 #pragma unroll
         for (int j = 0; j < 2; ++j) vaddr[j] = vofs[j] + sb;
-        const int64_t j0 = (tb + t) * BKV;
+        const int64_t j0 = (tb + T) * BKV;
 
         // S^T for the tile's two 32-key blocks. Step i of the 2 KS MFMAs is
         // key block i % 2, head-dim step i / 2 (two independent accumulation
@@ -415,8 +423,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention
         constexpr int NS = 2 * KS, G = D == 64 ? 8 : 4;
         constexpr int OPG = 2 * L::COPIES / (NS / G);   // tile t + 1 copies per MFMA group
         static_assert(OPG * (NS / G) == 2 * L::COPIES, "copies spread evenly over the groups");
-        const bool next = t + 1 < ntiles;
-        const __amdgpu_buffer_rsrc_t rkn = rsrc(t + 1, kh0), rvn = rsrc(t + 1, vh0);
+        const bool next = T + KG < ntiles;
+        const __amdgpu_buffer_rsrc_t rkn = rsrc(T + KG, kh0), rvn = rsrc(T + KG, vh0);
         LDS_AS char* nst = lds + ((t + 1) & 1) * L::STAGE + wave * L::COPIES * 1024;
         float16v sacc[2] = {(float16v)0.f, (float16v)0.f};
         half8 ka[2][G];
@@ -548,9 +556,41 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void attention
             for (int d = 0; d < DF; ++d)
                 o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vb[cur][d], pb[kk], o[d], 0, 0, 0);
         });
+        }
         // every wave is done reading stage t & 1 before tile t + 2 overwrites it
         __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));   // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
+    }
+
+    if constexpr (KG == 2) {
+        // (the last tile's barrier: every wave is done with both groups' stages)
+        LDS_AS char* all = (LDS_AS char*)(LDS_AS void*)fa_lds;
+        LDS_AS float4v* po = (LDS_AS float4v*)(all + L::BYTES + wave * (QW * D * 4)) + lane;
+        typedef float float2v __attribute__((ext_vector_type(2)));
+        LDS_AS float2v* pm = (LDS_AS float2v*)(all + wave * (QW * D * 4)) + lane;   // within wave's own rows below
+        if (kg == 1) {
+            *pm = float2v{m, l};
+#pragma unroll
+            for (int d = 0; d < DF; ++d)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4)
+                    po[(d * 4 + q4) * 64] = float4v{o[d][4 * q4], o[d][4 * q4 + 1], o[d][4 * q4 + 2], o[d][4 * q4 + 3]};
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        const float2v ml = *pm;
+        const float mm = fmaxf(m, ml[0]), mr = mm == -__builtin_inff() ? 0.f : mm;
+        const float a0 = __builtin_amdgcn_exp2f(m - mr), a1 = __builtin_amdgcn_exp2f(ml[0] - mr);
+        l = l * a0 + ml[1] * a1;
+        m = mm;
+#pragma unroll
+        for (int d = 0; d < DF; ++d)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const float4v v = po[(d * 4 + q4) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[d][4 * q4 + e] = o[d][4 * q4 + e] * a0 + v[e] * a1;
+            }
     }
 
     // Output: a partial when the key range is split, else O / l. A partial
@@ -877,6 +917,29 @@ static void flash_split(AttnParams& p, uint32_t cus)
     }
 }
 
+// Two wave groups per workgroup (D <= 128) where a CU has one workgroup, from
+// walks of 4 tiles up (16 heads over 2, D = 128, 2048 tokens 45.6 us with four
+// waves, 38.7 with eight; 32 x 64 x 1024 20.3, 16.2; chunks of 2 tiles 11.2,
+// 11.7), and up to two a CU where the walks are of unlike length, the longest
+// of which decides (causal 24 x 128 x 1500 36.3, 28.4; 12 x 64 x 4096 63.3, 46.3;
+// with even walks two workgroups of four waves overlap as well and need no
+// exchange: the same without a mask 48.7, 55.6). From three a CU on they tie.
+static uint32_t flash_key_groups(const AttnParams& p, uint32_t cus)
+{
+    const uint32_t nqt = (p.tq + fa::BQ - 1) / fa::BQ;
+    const uint64_t wgs = (uint64_t)(p.units ? p.units : nqt) * p.batch * p.hq;
+    if (p.dp > 128 || p.chunk_tiles < 4 || wgs > 2 * cus) return 1;
+    if (wgs <= cus) return 2;
+    int64_t sum = 0, longest = 0;   // (unsplit: a split is one round of at most cus)
+    for (uint32_t qt = 0; qt < nqt; ++qt) {
+        int64_t tb, te;
+        fa_tile_range(p, qt, plan_cached(p), tb, te);
+        sum += te - tb;
+        longest = std::max(longest, te - tb);
+    }
+    return 4 * sum <= 3 * longest * nqt ? 2 : 1;
+}
+
 // The split launch's tables: the units of a head, from the last query tile
 // (the longest causal walks start first), chunk by chunk; workgroup w -> unit
 // of head and batch, a head's units on one XCD.
@@ -933,6 +996,7 @@ void attention_plan(AttnParams& p, uint32_t cus)
     flash_split(p, cus);
     attention_decode_plan(p, cus, plan_cached(p) + p.tkv, flash_workspace(p));
     if (p.dec_units == 0 && p.units) flash_tables(p);
+    p.key_groups = flash_key_groups(p, cus);
 }
 
 // (the decode kernel's plan keeps within what the flash plan asks for)
@@ -953,17 +1017,17 @@ bool attention_ok(const AttnParams& p)
            dt_ok(p.q_dtype) && dt_ok(p.kv_dtype) && dt_ok(p.o_dtype);
 }
 
-template <int D>
+template <int D, int KG>
 static hipError_t attention_launch_d(const AttnParams& p, hipStream_t s)
 {
     static PerDevice lds_once;
     {
-        hipError_t e = set_max_lds(lds_once, (const void*)attention_fwd_kernel<D>, fa::Lds<D>::BYTES);
+        hipError_t e = set_max_lds(lds_once, (const void*)attention_fwd_kernel<D, KG>, KG * fa::Lds<D>::BYTES);
         if (e != hipSuccess) return e;
     }
     const uint32_t nqt = (p.tq + fa::BQ - 1) / fa::BQ;
     const dim3 grid = p.units ? dim3(p.units * p.hq * p.batch) : dim3(nqt, p.hq, p.batch);
-    hipLaunchKernelGGL(attention_fwd_kernel<D>, grid, dim3(256), fa::Lds<D>::BYTES, s, p);
+    hipLaunchKernelGGL((attention_fwd_kernel<D, KG>), grid, dim3(256 * KG), KG * fa::Lds<D>::BYTES, s, p);
     if (p.units == 0) return hipGetLastError();
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1001,10 +1065,11 @@ hipError_t attention_launch(const AttnParams& p0, hipStream_t s)
         p.v = v16;
         p.kv_dtype = DT_F16;
     }
+    const bool two = p.key_groups == 2;
     switch (p.dp) {
-    case 64: return attention_launch_d<64>(p, s);
-    case 128: return attention_launch_d<128>(p, s);
-    case 256: return attention_launch_d<256>(p, s);
+    case 64: return two ? attention_launch_d<64, 2>(p, s) : attention_launch_d<64, 1>(p, s);
+    case 128: return two ? attention_launch_d<128, 2>(p, s) : attention_launch_d<128, 1>(p, s);
+    case 256: return attention_launch_d<256, 1>(p, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -195,6 +195,7 @@ struct AttnParams {
     // (max, sum) go to ws_o / ws_ml and a merge pass combines them, finding
     // each query tile's first unit and chunk count in qt_tab.
     uint32_t units, chunk_tiles;
+    uint32_t key_groups;          // wave groups that take a workgroup's key tiles in turn (1 or 2)
     float* ws_o;                  // [batch*hq*units][128][dp] (fp32, or fp16 O / l for fp16 output)
     float* ws_ml;                 // [batch*hq*units][128][2]
     void* ws_kv;                  // fp16 copies of fp32 K then V (flash path), else null
