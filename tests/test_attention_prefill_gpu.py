@@ -57,3 +57,27 @@ def test_prefill(gpu, b, hq, hkv, tq, tkv, d, causal, span, odt):
             r = got[bb, :, h]
             assert np.isfinite(r).all() and (np.abs(r - y) <= tol).all(), (h, float((np.abs(r - y) / tol).max()))
             assert (r[none] == 0).all()
+
+
+@pytest.mark.parametrize("hq, hkv, t, d", [(2, 1, 200, 64), (24, 8, 1400, 128), (3, 3, 300, 256)])
+def test_prefill_nan_key(gpu, hq, hkv, t, d):
+    """A NaN score makes its own row NaN and no other: the rows before the key
+    (they may share a wave, and so the moves of the running maximum, with NaN
+    rows) stay within two roundings of P to fp16, other KV heads keep their bits."""
+    rng = np.random.default_rng(t)
+    q, k, v = (draw((1, h, t, d), rng, F16) for h in (hq, hkv, hkv))
+    D = gpu.DeviceArray.from_numpy
+    outs = []
+    j = t // 2 + 3
+    for bad in (False, True):
+        if bad:
+            k[0, 0, j, 5] = np.nan
+        out = gpu.DeviceArray((1, t, hq, d), F32)
+        out.fill_(0xFF)
+        print(f"prefill nan={bad} hq={hq} t={t} d={d}", flush=True)
+        outs.append(gpu.attention(out, D(q), D(k), D(v), causal=True).numpy())
+    g = hq // hkv
+    assert np.isfinite(outs[0]).all()
+    assert np.isnan(outs[1][0, j:, :g]).all()
+    assert np.allclose(outs[1][0, :j], outs[0][0, :j], rtol=0, atol=2.0 ** -10 * np.abs(v.astype(F32)).max())
+    assert (outs[1][0, :, g:] == outs[0][0, :, g:]).all()

@@ -111,13 +111,16 @@ __device__ __forceinline__ float fa_scale_acc(float x, float a)
     return x;
 }
 
-// Maximum of three (fmaxf keeps a quieting v_max per operand that comes from a
-// matrix core: 46 instructions for a tile's 32 scores instead of 16).
+// Maximum of three, as v_maximum3_f32 (fmaxf keeps a quieting v_max per operand
+// that comes from a matrix core: 46 instructions for a tile's 32 scores instead
+// of 16). A builtin and not inline asm: its operands are MFMA results, and only
+// for an instruction that the compiler itself places does it insert the wait
+// states between an MFMA and a vector read of its result. A NaN score gives a
+// NaN maximum, which moves no reference below; the row is NaN through its
+// exponential either way.
 __device__ __forceinline__ float fa_max3(float a, float b, float c)
 {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 
 template <int N>
