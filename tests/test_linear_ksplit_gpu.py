@@ -128,3 +128,52 @@ def test_ksplit_packed_weight(gpu, m, k, n, gated, tile):
         gpu.synchronize()
     got, want = outs[1].numpy(), outs[0].numpy()
     assert np.isfinite(got).all() and (got == want).all()
+
+
+def chain_error(k, step, chain, n=4096):
+    """Relative error (2-norm) of fp32 sums of k normal products, added `step` at a time to chains of `chain` k
+    whose totals are added in turn."""
+    rng = np.random.default_rng(k)
+    parts = rng.standard_normal((k // step, n)) * np.sqrt(step)   # one step's products, summed exactly
+    total = np.zeros(n, F32)
+    for c in range(0, k // step, chain // step):
+        run = np.zeros(n, F32)
+        for p in parts[c:c + chain // step].astype(F32):
+            run += p
+        total += run
+    want = parts.astype(F32).astype(np.float64).sum(axis=0)
+    return float(np.linalg.norm(total - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("m, k, n, xdt, tile, kw", [
+    (500, 4096, 4096, F16, "64x128", {}),
+    (400, 8192, 8192, F16, "128x128", {}),
+    (300, 8192, 2048, F16, "64x64", {}),
+    (300, 8191, 2048, F16, "64x64", {}),           # through registers
+    (61, 8192, 5120, F16, "32x64", {}),
+    (64, 8192, 1024, F16, "32x32", {}),
+    (500, 4096, 4096, F32, "64x128", {}),
+    (64, 4095, 1000, F32, "32x32", {"wdt": F32}),
+])
+def test_ksplit_long_k(gpu, m, k, n, xdt, tile, kw):
+    """The sums run in chains of at most 256 k (512 in 128x128 tiles from K = 3584, 128 with fp32 weights), the
+    shortest that a K split had at these sizes: the error against float64 is that of such chains, with a matrix
+    instruction's k taken 8 (fp32: 1) at a time. One chain over K has 2.5 times as much at K = 4096, sums over
+    a sixteenth of K = 8192 1.1 times."""
+    wdt = kw.get("wdt", F16)
+    rng = np.random.default_rng(m + k + n)
+    w, x = draw(normal((n, k), 0.05), rng, wdt), draw((m, k), rng, F16).astype(xdt)
+    D = gpu.DeviceArray.from_numpy
+    out = gpu.DeviceArray((m, n), F32)
+    a = gpu.linear_args(out, D(x), D(w))
+    name = gpu.linear_plan(a)[0]
+    print(f"ksplit chains m={m} k={k} n={n} plan={name}", flush=True)
+    assert name == f"tile_f{8 * w.itemsize}_{tile}_kwaves"
+    gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
+    gpu.synchronize()
+    cols = slice(n // 2, n // 2 + 64)
+    want = x.astype(np.float64) @ w[cols].astype(np.float64).T
+    err = float(np.linalg.norm(out.numpy()[:, cols] - want) / np.linalg.norm(want))
+    bound = chain_error((k + 511) // 512 * 512, *((1, 128) if wdt == F32 else (8, 512 if tile == "128x128" else 256)))
+    print(f"  error {err:.2e}, chains {bound:.2e}", flush=True)
+    assert err <= 1.04 * bound

@@ -70,6 +70,16 @@ struct Cfg {
     static constexpr int KQ = F32 ? 8 : 16, KSTEPS = BK / KQ;
     // sums per output and wave (k steps in turn)
     static constexpr int AS = F32 ? (KSP ? 2 : 4) : !KSP ? 1 : WM * WN <= 32 * 64 ? (BK / 16 < 4 || NW == 8 ? 2 : 4) : 2;
+    // Long K: sums per output and wave (fewer where the total takes their
+    // registers), and the stages after which they go to the total: chains of at
+    // most 256 k (fp32: 128).
+    static constexpr int LAS = KSP && WM * WN == 32 * 64 ? (DMA ? 2 : 1) : WM * WN > 32 * 64 ? 1 : AS;
+    static constexpr int CHAIN = (F32 ? 128 : 256) * LAS / BK;
+    // The quadrants over fp16 X fit in 256 registers (accumulation registers would
+    // cost a move per element and chain); with fp32 X 128x128 would spill.
+    static constexpr int WPS = NW == 8 || (!KSP && DMA && sizeof(TA_) == 2) ? 2 : 1;
+    // whether a wave's share of K is longer than its sums' chains
+    static bool long_k(uint32_t K) { return K > (F32 ? 128u : 256u) * AS * (KSP ? NW : 1); }
     static constexpr int AES = DMA || F32 ? (int)sizeof(TA) : 2, BES = (int)sizeof(TB);   // element bytes in LDS
     static constexpr int AROW = BK * AES, BROW = BK * BES;       // row bytes in LDS
     static constexpr int ABYTES = BM * AROW, BBYTES = BN * BROW, STAGE = ABYTES + BBYTES;
@@ -106,8 +116,8 @@ __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 
 
 }   // namespace ks
 
-template <typename C, bool GATED>
-__global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_kernel(GemmParams p, const half_t* __restrict__ packed)
+template <typename C, bool GATED, bool LONG>
+__global__ __launch_bounds__(64 * C::NW, C::WPS) void gemm_ksplit_kernel(GemmParams p, const half_t* __restrict__ packed)
 {
     using namespace ks;
     constexpr int BM = C::BM, BN = C::BN, NW = C::NW, BK = C::BK, S = C::S;
@@ -309,22 +319,29 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
     }
 
     // D = W X^T: lane (fr, fk) holds X row i*32 + fr at columns j*32 + 8 g + 4 fk .. +3.
-    // The k steps go to AS sums in turn: with the waves' own K shares at
-    // least 8 shorter chains per output, as exact as a split-K launch with
-    // its planes summed (K = 4096: 1.3e-7 relative; one chain a wave 1.6e-7).
-    constexpr int AS = C::AS;
-    float16v acc[AS][FM][FN];
+    // The k steps go to AS sums in turn. LONG: no sum runs over more than 256 k
+    // (fp32 128), the shortest split of the split-K launches whose place this
+    // kernel takes, before it goes to the total, so that the error is no larger
+    // than theirs (K = 4096: one chain 4.1e-7 relative, 8 splits 1.6e-7, this
+    // 1.3e-7; K = 8192 in 16 sums 1.6e-7, this 1.3e-7). A chain's first MFMA
+    // starts from a zero operand; the additions run beside the MFMAs before it
+    // (fp16 X, us, one chain / this: [500, 4096], N 4096 31.8 / 32.8; [400,
+    // 4096], N 8192 42.5 / 45; [61, 8192], N 5120 21.9 / 22.3).
+    constexpr int AS = LONG ? C::LAS : C::AS;
+    float16v acc[AS][FM][FN], total[FM][FN];
 #pragma unroll
-    for (int a = 0; a < AS; ++a)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int j = 0; j < FN; ++j) {
+            total[i][j] = (float16v)0.f;
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[a][i][j] = (float16v)0.f;
+            for (int a = 0; a < AS; ++a) acc[a][i][j] = (float16v)0.f;
+        }
 
     // A stage's MFMAs; step(q) runs after those of k step q. KSP reads all of
     // the stage's fragments first (so that its slot can be refilled during the
-    // MFMAs), the shared ring's waves read one step ahead.
-    const auto stage_mfma = [&](const LDS_AS char* st, auto&& step) __attribute__((always_inline)) {
+    // MFMAs), the shared ring's waves read one step ahead. NEW: new chains start.
+    const auto stage_mfma = [&](const LDS_AS char* st, auto NEW, auto&& step) __attribute__((always_inline)) {
         constexpr int AHEAD = C::KSP ? KSTEPS : 1, SETS = C::KSP ? KSTEPS : 2;
         frag xf[SETS][FM], wf[SETS][FN];
 #pragma unroll
@@ -343,6 +360,12 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
                 for (int j = 0; j < FN; ++j) wf[(q + AHEAD) % SETS][j] = read_w(st, j, q + AHEAD);
             }
+            // the next MFMA of a sum: its chain so far, or nothing as that joins the total
+            const auto chain = [&](int a, int i, int j, bool first) __attribute__((always_inline)) {
+                if (!first) return acc[a][i][j];
+                total[i][j] += acc[a][i][j];
+                return (float16v)0.f;
+            };
             if constexpr (C::F32) {
                 // element e of both halves' pieces is one k pair (the same on both operands)
 #pragma unroll
@@ -352,18 +375,28 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
                         for (int j = 0; j < FN; ++j)
                             acc[e % AS][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                wf[q % SETS][j][e], xf[q % SETS][i][e], acc[e % AS][i][j], 0, 0, 0);
+                                wf[q % SETS][j][e], xf[q % SETS][i][e], chain(e % AS, i, j, NEW && q == 0 && e < AS), 0, 0, 0);
             } else {
 #pragma unroll
                 for (int i = 0; i < FM; ++i)
 #pragma unroll
                     for (int j = 0; j < FN; ++j)
-                        acc[q % AS][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[q % SETS][j], xf[q % SETS][i],
-                                                                                   acc[q % AS][i][j], 0, 0, 0);
+                        acc[q % AS][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            wf[q % SETS][j], xf[q % SETS][i], chain(q % AS, i, j, NEW && q < AS), 0, 0, 0);
             }
             if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
             step(q);
             if constexpr (C::DMA) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // stage(r, NEW) for r = 0 .. mine - 1
+    // (128x128 replaced at most 7 splits: 512 k and more each from K = 3584 up)
+    const uint32_t chain = C::CHAIN * (BM == 128 && K >= 7 * 512 ? 2u : 1u);
+    const auto stages = [&](auto&& stage) __attribute__((always_inline)) {
+        for (int r = 0; r < mine;) {
+            const int end = LONG ? std::min(r + (int)chain, mine) : mine;
+            if constexpr (LONG) stage(r++, std::true_type{});
+            for (; r < end; ++r) stage(r, std::false_type{});
         }
     };
 
@@ -375,13 +408,13 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
         for (int r = 0; r < S; ++r) issue(r, wave + r * NW);
         int slot = 0;
-        for (int r = 0; r < mine; ++r) {
+        stages([&](int r, auto NEW) __attribute__((always_inline)) {
             wait_vmcnt<(S - 1) * C::COPIES>();
-            stage_mfma(ring + slot * C::STAGE, [&](int q) __attribute__((always_inline)) {
+            stage_mfma(ring + slot * C::STAGE, NEW, [&](int q) __attribute__((always_inline)) {
                 issue_part(slot, wave + (r + S) * NW, q);
             });
             slot = slot + 1 == S ? 0 : slot + 1;
-        }
+        });
         wait_vmcnt<0>();   // the copies past the range land before LDS is reused
     } else if constexpr (C::DMA) {
         // Stages r .. r + S - 2 are issued at the top of trip r: once at most
@@ -392,41 +425,41 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
 #pragma unroll
         for (int r = 0; r < S - 1; ++r) issue(r, r);
         int slot = 0;
-        for (int r = 0; r < mine; ++r) {
+        stages([&](int r, auto NEW) __attribute__((always_inline)) {
             wait_vmcnt<(S - 2) * C::COPIES>();
             wait_lgkmcnt0();
             __builtin_amdgcn_s_barrier();
             const int free = slot == 0 ? S - 1 : slot - 1;
-            stage_mfma(ring + slot * C::STAGE,
+            stage_mfma(ring + slot * C::STAGE, NEW,
                        [&](int q) __attribute__((always_inline)) { issue_part(free, r + S - 1, q); });
             slot = slot + 1 == S ? 0 : slot + 1;
-        }
+        });
         wait_vmcnt<0>();   // the copies past the range land before LDS is reused
     } else if constexpr (C::KSP) {
         if (mine > 0) fetch(wave);
-        for (int r = 0; r < mine; ++r) {
+        stages([&](int r, auto NEW) __attribute__((always_inline)) {
             place(0);
             if (r + 1 < mine) fetch(wave + (r + 1) * NW);
-            stage_mfma(ring, [](int) {});
-        }
+            stage_mfma(ring, NEW, [](int) {});
+        });
     } else {
         // A wave that writes stage r + 2 has passed the barrier of trip
         // r + 1, so every wave is done reading stage r from the same slot.
         fetch(0);
-        for (int r = 0; r < mine; ++r) {
+        stages([&](int r, auto NEW) __attribute__((always_inline)) {
             place(r & 1);
             if (r + 1 < mine) fetch(r + 1);
             __syncthreads();
-            stage_mfma(ring + (r & 1) * C::STAGE, [](int) {});
-        }
+            stage_mfma(ring + (r & 1) * C::STAGE, NEW, [](int) {});
+        });
     }
 
 #pragma unroll
-    for (int a = 1; a < AS; ++a)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+        for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[0][i][j] += acc[a][i][j];
+            for (int a = 0; a < AS; ++a) total[i][j] += acc[a][i][j];
 
     // ---- the partial tiles meet in LDS, RB rows at a time ----
     // U rows of a thread's four columns at a time, the residual of the next U
@@ -466,7 +499,7 @@ __global__ __launch_bounds__(64 * C::NW, C::NW == 8 ? 2 : 1) void gemm_ksplit_ke
                 for (int g = 0; g < 4; ++g) {
                     const int row = (C::KSP ? wave * C::RB : wm0) + i * 32 + fr - h * C::RB;
                     *(LDS_AS float4v*)(lds + row * C::RROW + (wn0 + j * 32 + 8 * g + 4 * fk) * 4) =
-                        float4v{acc[0][i][j][4 * g], acc[0][i][j][4 * g + 1], acc[0][i][j][4 * g + 2], acc[0][i][j][4 * g + 3]};
+                        float4v{total[i][j][4 * g], total[i][j][4 * g + 1], total[i][j][4 * g + 2], total[i][j][4 * g + 3]};
                 }
         __syncthreads();
         const auto sums = [&](uint32_t rr, float4v& v, float4v& up) __attribute__((always_inline)) {
@@ -613,16 +646,32 @@ int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
     return best;
 }
 
+template <typename C, bool GATED, bool LONG>
+static hipError_t launch_long(const GemmParams& p, const void* packed, hipStream_t s)
+{
+    static PerDevice lds_once;
+    hipError_t e = set_max_lds(lds_once, (const void*)gemm_ksplit_kernel<C, GATED, LONG>, C::LDS);
+    if (e != hipSuccess) return e;
+    const uint32_t no = GATED ? p.H : p.N, bno = GATED ? C::BN / 2 : C::BN;
+    const uint32_t tiles = ((p.M + C::BM - 1) / C::BM) * ((no + bno - 1) / bno);
+    hipLaunchKernelGGL((gemm_ksplit_kernel<C, GATED, LONG>), dim3(tiles), dim3(64 * C::NW), C::LDS, s, p,
+                       (const half_t*)packed);
+    return hipGetLastError();
+}
+
 template <typename C, bool GATED>
 static hipError_t launch_cfg(const GemmParams& p, const void* packed, hipStream_t s)
 {
-    static PerDevice lds_once;
-    hipError_t e = set_max_lds(lds_once, (const void*)gemm_ksplit_kernel<C, GATED>, C::LDS);
-    if (e != hipSuccess) return e;
-    const uint32_t no = GATED ? p.H : p.N, bno = GATED ? C::BN / 2 : C::BN;
-    const uint32_t tiles = ((p.M + C::BM - 1) / C::BM) * ((no + bno - 1) / bno) ;
-    hipLaunchKernelGGL((gemm_ksplit_kernel<C, GATED>), dim3(tiles), dim3(64 * C::NW), C::LDS, s, p, (const half_t*)packed);
-    return hipGetLastError();
+    // (an fp16 quadrant's one sum is 256 k long at once; fp32 quadrants keep four
+    // sums, more than the splits the same sizes had: they take 61 and more tiles
+    // of 64x64, and so at most 4)
+    if constexpr (C::F32 && !C::KSP) {
+        return launch_long<C, GATED, false>(p, packed, s);
+    } else {
+        if constexpr (C::KSP)
+            if (!C::long_k(p.K)) return launch_long<C, GATED, false>(p, packed, s);
+        return launch_long<C, GATED, true>(p, packed, s);
+    }
 }
 
 template <typename TA, bool DMA, bool PK, bool GATED>
