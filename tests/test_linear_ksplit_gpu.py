@@ -177,3 +177,38 @@ def test_ksplit_long_k(gpu, m, k, n, xdt, tile, kw):
     bound = chain_error((k + 511) // 512 * 512, *((1, 128) if wdt == F32 else (8, 512 if tile == "128x128" else 256)))
     print(f"  error {err:.2e}, chains {bound:.2e}", flush=True)
     assert err <= 1.04 * bound
+
+
+@pytest.mark.parametrize("m, k, n, xdt, wdt, off, tile", [
+    (22, 7864, 256, F32, F32, 0, "64x64"),
+    (9, 4095, 130, F32, F32, 0, "64x64"),
+    (40, 8200, 96, F32, F16, 0, "64x64"),
+    (33, 16384, 40, F16, F16, 1, "64x64"),
+])
+def test_long_k_over_few_tiles(gpu, m, k, n, xdt, wdt, off, tile):
+    """K split over workgroups where the small tiles are too few for the chip; without the workspace for that
+    (or with one too small) the small tiles run."""
+    rng = np.random.default_rng(k)
+    w, x = draw(normal((n, k), 0.05), rng, wdt), draw((m, k), rng, F16).astype(xdt)
+    D = gpu.DeviceArray.from_numpy
+    dw = D(np.concatenate([np.zeros(off, wdt), w.ravel()]))
+    out = gpu.DeviceArray((m, n), F32)
+    a = gpu.linear_args(out, D(x), D(w))
+    a.weight = dw.ptr + w.itemsize * off
+    name, splits = gpu.linear_plan(a)
+    need = gpu.linear_workspace_size(a)
+    print(f"few tiles m={m} k={k} n={n} plan={name} splits={splits}", flush=True)
+    assert name == f"tile_f{8 * w.itemsize}_{tile}" and splits > 1 and need == splits * m * n * 4
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    want, tol = x64 @ w64.T, (np.abs(x64) @ np.abs(w64).T) * (k + 1) * 2.0 ** -24
+    ws = gpu.DeviceArray((need,), np.uint8)
+    errs = []
+    for ptr, size in ((ws.ptr, need), (None, 0), (ws.ptr, need - 4)):
+        out.fill_(0xFF)
+        a.workspace, a.workspace_bytes = ptr, size
+        gpu.check(gpu.lib().vai_linear_launch(ctypes.byref(a), None), "linear")
+        gpu.synchronize()
+        got = out.numpy().astype(np.float64)
+        assert np.isfinite(got).all() and (np.abs(got - want) <= tol).all()
+        errs.append(got)
+    assert (errs[1] == errs[2]).all()

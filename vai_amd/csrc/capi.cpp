@@ -36,7 +36,8 @@ vai_status hip_status(hipError_t e) { return e == hipSuccess ? VAI_OK : (vai_sta
 
 struct LinearPlan {
     enum Kind { Slab, SlabThenGate, Tile, BigTile, PackedTile, F32Small, Acc16Tile, KSplit } kind;
-    int ks_tile;        // KSplit: which tile
+    int ks_tile;        // KSplit (or with ks_spare): which tile
+    bool ks_spare;      // Tile, PackedTile: the small tiles take a launch without the workspace
     bool packed_gemv;   // Slab / SlabThenGate over the packed weight
     GemmTile tile;
     uint32_t bm, bn;
@@ -122,6 +123,72 @@ float packed_us(const GemmParams& g, bool gated, uint32_t tiles)
     return S == 1 ? us : us + 4.f + (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 4e6f;
 }
 
+// The generic tiles, with a K split where even the smallest leave CUs idle.
+LinearPlan plan_tile(const vai_linear_args* a)
+{
+    LinearPlan p{};
+    p.kind = LinearPlan::Tile;
+    const uint32_t M = a->M, N = a->N, K = a->K;
+    const bool f32 = a->i_dtype == VAI_DTYPE_F32 && a->w_dtype == VAI_DTYPE_F32;
+    const uint32_t bk = f32 ? 16 : 32;
+    // Candidate tiles, largest first (the gated kernel pairs fragments, so its
+    // smallest N tile is 128 columns = 64 output columns).
+    struct Cand { GemmTile t; uint32_t bm, bn; };
+    const Cand cands[] = {
+        {GemmTile::T256x128, 256, 128}, {GemmTile::T128x128, 128, 128},
+        {GemmTile::T128x64, 128, a->gated ? 128u : 64u}, {GemmTile::T64x64, 64, a->gated ? 128u : 64u},
+    };
+    const uint32_t ncols = N;   // gated: 2H logical columns
+    Cand pick = cands[3];
+    for (const Cand& c : cands) {
+        if (f32 && c.bm == 256) continue;   // fp32 staging keeps 128-row tiles (LDS, registers)
+        if (tiles_of(M, ncols, c.bm, c.bn) >= plan_cus()) { pick = c; break; }
+    }
+    p.tile = pick.t;
+    p.bm = pick.bm;
+    p.bn = pick.bn;
+    const uint32_t tiles = tiles_of(M, ncols, pick.bm, pick.bn);
+    if (a->split_size) {
+        p.split_size = a->split_size;
+        p.splits = (K + a->split_size - 1) / a->split_size;
+    } else {
+        uint32_t splits = 1;
+        if (f32 && tiles < plan_cus() && K >= 256) {
+            // fp32 matrix cores run at 1/16 of the fp16 rate, so a small fp32
+            // GEMM is bound by how many SIMDs it keeps busy: aim at ~1.5
+            // workgroups per CU (config 1, 96 tiles, K 768: 4 splits, 19 us,
+            // against 36.7 us unsplit and 21 us with 3 or 6 splits)
+            splits = std::min<uint32_t>((3 * plan_cus() / 2 + tiles / 2) / tiles, K / 128);
+            splits = std::max<uint32_t>(splits, 1);
+        } else if (tiles < plan_cus() / 2 && K >= 1024) {
+            splits = std::min<uint32_t>((plan_cus() + tiles - 1) / tiles, K / 256);
+            splits = std::max<uint32_t>(splits, 1);
+        }
+        p.split_size = splits > 1 ? ((K + splits - 1) / splits + bk - 1) / bk * bk : K;
+        p.splits = (K + p.split_size - 1) / p.split_size;
+    }
+    p.workspace = p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+    return p;
+}
+
+// The generic tiles' time (us) with a K split: a launch and the k of one split
+// (rows that are not whole aligned vectors load their elements singly), and the
+// reduce pass, which adds the planes in turn. Against it the small tiles' time
+// on the few CUs that these sizes give them (gemm_ksplit_few_us). Measured, us,
+// split / small tiles: X fp32 [64, 4096], N 64 15.0 / 12.2; [32, 6144] 15.1 /
+// 16.5; [64, 32768], N 512 46.9 / 102; X fp16 [64, 16384], N 256 26.9 / 21.3;
+// [64, 32768] 33.8 / 40; fp32 W, K 2047, N 256, 64 rows 16.2 / 14; K 4095 20.7 /
+// 23.4; K 7864 25.9 / 37.2.
+float split_us(const GemmParams& g, uint32_t S)
+{
+    const float planes = (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 2e6f;
+    const bool aligned = (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
+    if (g.b_dtype == VAI_DTYPE_F32)
+        return 2.f + .265f * (float)S + (g.K % 4 == 0 && aligned ? .062f : .08f) * (float)(g.K / S) + planes;
+    return 3.f + (aligned ? .3f : .27f) * (float)S +
+           (g.K % 8 != 0 ? .11f : aligned ? .028f : .05f) * (float)(g.K / S) + planes;
+}
+
 LinearPlan plan_linear(const vai_linear_args* a)
 {
     LinearPlan p{};
@@ -180,6 +247,9 @@ LinearPlan plan_linear(const vai_linear_args* a)
             const bool small = M < 512 || splits > 8;
             if (gemm_packed_ok(g, a->gated) && !(small && ksplit && ksplit_us < packed_us(g, a->gated != 0, tiles))) {
                 p.kind = LinearPlan::PackedTile;
+                // (an X off a 16-byte boundary can move a call here that asked
+                // for its workspace with an aligned one, which needs none)
+                p.ks_spare = small && ksplit;
                 p.splits = splits;
                 p.split_size = K / splits;
                 p.workspace = splits > 1 ? (size_t)splits * M * N * 4 : 0;
@@ -204,6 +274,17 @@ LinearPlan plan_linear(const vai_linear_args* a)
             return p;
         }
         if (ksplit && !(M >= 512 && gemm_big_ok(g, a->gated))) {
+            // a long K over few tiles: split over workgroups, where that is
+            // faster and its planes fit the library's own scratch too
+            if (!a->gated) {
+                LinearPlan t = plan_tile(a);
+                if (t.splits > 1 && t.workspace <= VAI_NOALLOC_SCRATCH_BYTES &&
+                    split_us(g, t.splits) < gemm_ksplit_few_us(g)) {
+                    t.ks_tile = p.ks_tile;
+                    t.ks_spare = true;
+                    return t;
+                }
+            }
             p.kind = LinearPlan::KSplit;
             p.splits = 1;
             p.split_size = K;
@@ -218,46 +299,7 @@ LinearPlan plan_linear(const vai_linear_args* a)
             return p;
         }
     }
-    const bool f32 = a->i_dtype == VAI_DTYPE_F32 && a->w_dtype == VAI_DTYPE_F32;
-    const uint32_t bk = f32 ? 16 : 32;
-    // Candidate tiles, largest first (the gated kernel pairs fragments, so its
-    // smallest N tile is 128 columns = 64 output columns).
-    struct Cand { GemmTile t; uint32_t bm, bn; };
-    const Cand cands[] = {
-        {GemmTile::T256x128, 256, 128}, {GemmTile::T128x128, 128, 128},
-        {GemmTile::T128x64, 128, a->gated ? 128u : 64u}, {GemmTile::T64x64, 64, a->gated ? 128u : 64u},
-    };
-    const uint32_t ncols = N;   // gated: 2H logical columns
-    Cand pick = cands[3];
-    for (const Cand& c : cands) {
-        if (f32 && c.bm == 256) continue;   // fp32 staging keeps 128-row tiles (LDS, registers)
-        if (tiles_of(M, ncols, c.bm, c.bn) >= plan_cus()) { pick = c; break; }
-    }
-    p.tile = pick.t;
-    p.bm = pick.bm;
-    p.bn = pick.bn;
-    const uint32_t tiles = tiles_of(M, ncols, pick.bm, pick.bn);
-    if (a->split_size) {
-        p.split_size = a->split_size;
-        p.splits = (K + a->split_size - 1) / a->split_size;
-    } else {
-        uint32_t splits = 1;
-        if (f32 && tiles < plan_cus() && K >= 256) {
-            // fp32 matrix cores run at 1/16 of the fp16 rate, so a small fp32
-            // GEMM is bound by how many SIMDs it keeps busy: aim at ~1.5
-            // workgroups per CU (config 1, 96 tiles, K 768: 4 splits, 19 us,
-            // against 36.7 us unsplit and 21 us with 3 or 6 splits)
-            splits = std::min<uint32_t>((3 * plan_cus() / 2 + tiles / 2) / tiles, K / 128);
-            splits = std::max<uint32_t>(splits, 1);
-        } else if (tiles < plan_cus() / 2 && K >= 1024) {
-            splits = std::min<uint32_t>((plan_cus() + tiles - 1) / tiles, K / 256);
-            splits = std::max<uint32_t>(splits, 1);
-        }
-        p.split_size = splits > 1 ? ((K + splits - 1) / splits + bk - 1) / bk * bk : K;
-        p.splits = (K + p.split_size - 1) / p.split_size;
-    }
-    p.workspace = p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
-    return p;
+    return plan_tile(a);
 }
 
 const char* tile_name(GemmTile t, bool gated)
@@ -392,8 +434,13 @@ vai_status vai_linear_launch(const vai_linear_args* a, vai_stream_t stream)
 {
     const vai_status st = check_linear(a);
     if (st != VAI_OK) return st;
-    const LinearPlan p = plan_linear(a);
-    if (p.workspace && (!a->workspace || a->workspace_bytes < p.workspace)) return VAI_ERR_WORKSPACE;
+    LinearPlan p = plan_linear(a);
+    if (p.workspace && (!a->workspace || a->workspace_bytes < p.workspace)) {
+        if (!p.ks_spare) return VAI_ERR_WORKSPACE;
+        p.kind = LinearPlan::KSplit;
+        p.splits = 1;
+        p.split_size = a->K;
+    }
     return linear_run(a, p, (hipStream_t)stream);
 }
 

@@ -646,6 +646,19 @@ int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
     return best;
 }
 
+// The 32x32 tile's time where its tiles are far fewer than the CUs: more bytes a
+// cycle for each than on a full grid (8 and 32 tiles, K = 2048 to 32768; fp32
+// operands alike).
+float gemm_ksplit_few_us(const GemmParams& p)
+{
+    const float chunks = (float)((p.K + 63) / 64);
+    if (p.b_dtype == DT_F32) return 4.f + .31f * chunks;
+    // (fp32 X in rows off 128-byte lines: 234 x 7080 25.3 us)
+    if (p.a_dtype == DT_F32)
+        return 4.2f + (!ks::dma_ok(p) ? .16f : p.K % 32 == 0 || p.M <= 32 ? .135f : .175f) * chunks;
+    return 4.7f + (ks::dma_ok(p) ? .08f : .125f) * chunks;
+}
+
 template <typename C, bool GATED, bool LONG>
 static hipError_t launch_long(const GemmParams& p, const void* packed, hipStream_t s)
 {
