@@ -81,8 +81,11 @@ def test_plans():
     assert splits == 4
     name, splits = plan(2048, 16384, 3072, gated=1, gate_epilogue=4)
     assert name.endswith("_gated") and splits == 1
-    # few small tiles: over a long K split among workgroups, over a short one not
+    # fp32, many rounds of 16-column tiles
     f32 = dict(idt=np.float32, wdt=np.float32)
+    assert plan(524, 5832, 6656, **f32)[0] == "tile_f32_32x32_kwaves"
+    assert plan(512, 3072, 768, **f32)[0] == "tile_f32_32x48_kwaves"
+    # few small tiles: over a long K split among workgroups, over a short one not
     assert plan(22, 256, 7864, **f32)[1] > 1 and plan(22, 256, 1100, **f32)[1] == 1
     assert plan(64, 64, 8192, np.float32)[1] > 1 and plan(64, 64, 2048, np.float32)[1] == 1
     assert plan(64, 1024, 8192)[1] == 1

@@ -259,10 +259,14 @@ LinearPlan plan_linear(const vai_linear_args* a)
         }
         // fp32 problems with fewer 64x64 tiles than CUs, or where its rounds of
         // 32-row tiles still take less: one launch over the full K with a
-        // CU-filling tile count
+        // CU-filling tile count. Over more than 16 rounds of 16 columns the
+        // operands' repeated reads count: 17 to 25 rounds of K = 4736 to 7424 took
+        // 1.1-1.8 times the model ([524, 6656], N 5832 714 us; in 32x32 tiles,
+        // whose sums are as exact, 411).
         const int nf = gemm_f32_nf(M, N, plan_cus());
-        const float f32_us = 2.5f + (float)((tiles_of(M, N, 32, 16 * nf) + plan_cus() - 1) / plan_cus()) *
-                                        (2.f + 0.0022f * (float)nf * (float)K);
+        const uint32_t rounds = (tiles_of(M, N, 32, 16 * nf) + plan_cus() - 1) / plan_cus();
+        float f32_us = 2.5f + (float)rounds * (2.f + 0.0022f * (float)nf * (float)K);
+        if (nf == 1 && rounds > 16 && p.ks_tile == 0) f32_us *= 1.3f;
         if (a->split_size == 0 && !a->gated && gemm_f32_ok(g) &&
             (tiles_of(M, N, 64, 64) < plan_cus() || !ksplit || f32_us <= ksplit_us)) {
             p.kind = LinearPlan::F32Small;
