@@ -80,3 +80,24 @@ def test_conv_direct(gpu, b, ci, co, h, w, k, stride, xdt, odt, epi, residual, o
     tol = 1.2 * tol + 2e-6 * np.abs(y) + (2.0 ** -11 * np.abs(y) if odt == F16 else 0)   # slopes up to 1.13
     got = out.numpy().astype(np.float64)
     assert np.isfinite(got).all() and (np.abs(got - y) <= tol).all(), float((np.abs(got - y) / tol).max())
+
+
+@pytest.mark.parametrize("xdt, w", [(F16, 136), (F32, 136), (F16, 141)])
+def test_conv_direct_infinite_weight(gpu, xdt, w):
+    """An infinite weight of a full channel block reaches its own output once: the last block, of one octet where
+    the one before has 44, does not multiply it by the zeros of the channels that it lacks."""
+    ci, co, h, bad = 360, 64, 5, 200
+    rng = np.random.default_rng(w)
+    x, wt = draw(lambda g: g.uniform(0.5, 1, (1, ci, h, w)), rng, xdt), draw(normal((co, ci, 1, 1), 0.1), rng, F16)
+    wt[7, bad] = np.inf
+    D = gpu.DeviceArray.from_numpy
+    out = gpu.DeviceArray((1, co, h, w), F32)
+    out.fill_(0xFF)
+    print(f"conv direct infinity {np.dtype(xdt)} w={w}", flush=True)
+    got = gpu.conv2d(out, D(x), D(wt)).numpy()
+    x64, w64 = x.astype(np.float64), wt.astype(np.float64)
+    assert (got[0, 7] == np.inf).all()
+    keep = np.arange(co) != 7
+    mag = conv64(np.abs(x64), np.abs(w64[keep]), 1)
+    tol = mag * (ci * 2.0 ** -24 + (2.0 ** -11 if xdt == F32 else 0)) + 1e-6
+    assert (np.abs(got[:, keep] - conv64(x64, w64[keep], 1)) <= tol).all()

@@ -156,8 +156,10 @@ __global__ __launch_bounds__(cd::NT, 4) void conv_direct_kernel(ConvDirectParams
             }
         };
         load_w(tid);
-        // the weights' padding (octets past the block, channels past Ci) is zero
-        if (q.oct4 != q.oct || cn % 8) {
+        // the weights' padding is zero: octets past the block, channels past Ci,
+        // and in a short last block what the block before left (its infinities
+        // must not meet the zeros of the window)
+        if (q.oct4 != q.oct || cn % 8 || cn != q.cb) {
             for (uint32_t i = tid; i < CT * q.wu; i += NT) *(LDS_AS half8*)(win + i * 16) = (half8)(half_t)0;
             __syncthreads();
         }
