@@ -61,6 +61,12 @@ def test_slab_any(gpu, m, k, n, xdt, wdt, odt, off, plan="slab_scalar"):
     (6, 1028, 2049, F32, F32, F32),       # ... and X through LDS
     (4, 1032, 1030, F32, F16, F32),
     (3, 516, 17, F32, F32, F32),
+    (4, 3504, 3075, F32, F16, F32),       # three and four rows staged in LDS: long rows ...
+    (3, 2052, 12291, F32, F32, F16),
+    (4, 1000, 33, F32, F32, F32),         # ... and rows of one K block
+    (5, 600, 2049, F32, F32, F32),
+    (8, 516, 2060, F16, F32, F32),
+    (7, 4096, 1537, F32, F32, F32),
 ])
 def test_slab_whole_chunks(gpu, m, k, n, xdt, wdt, odt):
     """Rows of whole chunks with more activations than a lane holds ahead."""

@@ -216,11 +216,9 @@ __global__ __launch_bounds__(256) void slab_reg_kernel(const TW* __restrict__ Wp
 }
 
 
-// 5-8 input rows against many long fp32 rows: the M rows of each K block are
-// staged once per workgroup in LDS and broadcast to the four waves (the X of
-// each wave would be twice its W bytes: K = 2048, N = 4096 11.3 us, 11.6-12.7
-// without; below, the barriers cost more: K = 768, N = 3072 5.7 against 4.8,
-// K = 3072, N = 768 11.0 against 7.2).
+// 3-8 input rows where their bytes, read from L2 by every wave, cost more than
+// a barrier does (staged_x): the M rows of each K block are staged once per
+// workgroup in LDS and broadcast to the four waves.
 template <int MP, int R, int KCH, typename TI, typename TW>
 __global__ __launch_bounds__(256) void slab_vec_kernel(SlabParams a)
 {
@@ -486,6 +484,28 @@ static hipError_t launch_any(const SlabParams& a, hipStream_t s)
     return go(std::integral_constant<int, 1>{});
 }
 
+// Which of the calls with more activations than a lane holds ahead stage X in
+// LDS (slab_vec_kernel) and which read it from L2 (slab_any_kernel). Measured,
+// us, staged / from L2. Long and many rows, where a wave reads twice the bytes
+// of its W as X: X fp32, W fp16, 4 rows, K = 4096, N = 16384 29.6 / 36.9, K = 8192,
+// N = 32768 99 / 186, but K = 6400, N = 6144 21.8 / 20.2, K = 2048, N = 4096 8.3 /
+// 7.6; W fp32, 4 rows, K = 6400, N = 16384 65 / 86, 8 rows, K = 2048, N = 4096 11.3 /
+// 11.6-12.7, but N = 1024 8.1 / 7.3. fp32 rows of one K block (512 to 1024
+// elements), which are read from L2 in three or four passes: 5 rows, K = 1000, N =
+// 2048 4.5 / 5.5, 4 rows, N = 8192 7.3 / 8.6, but 5 rows, K = 768, N = 8192 8.7 / 7.8.
+template <int MP, typename TI, typename TW>
+static bool staged_x(uint32_t K, uint32_t N)
+{
+    constexpr bool x32 = sizeof(TI) == 4, w32 = sizeof(TW) == 4;
+    if (MP == 4) {
+        if (!w32) return K >= 3500 && N >= (K < 4608 ? 3072u : K < 8192 ? 16384u : 6144u);
+        return (K > 768 && K < 1024) || (K >= 2048 && N >= 12288);
+    }
+    if (!w32) return false;
+    if (N >= 2048 && K > 512) return K >= 1024 || N < (x32 ? 8192u : 3072u);
+    return x32 && K >= 1024 && N >= 1536 && (uint64_t)N * K >= 5500000;
+}
+
 template <int MP, typename TI, typename TW>
 static hipError_t launch_vec(const SlabParams& a, hipStream_t s)
 {
@@ -504,15 +524,15 @@ static hipError_t launch_vec(const SlabParams& a, hipStream_t s)
                                (const TW*)a.weight, (const TI*)a.in, a.K, a.N, a.M, a);
         return hipGetLastError();
     } else {
-        if constexpr (MP == 8 && sizeof(TW) == 4)
-            if (a.N >= 2048 && a.K >= 1024) {
-                hipLaunchKernelGGL((slab_vec_kernel<MP, R, KCH, TI, TW>), dim3(blocks), dim3(256), 0, s, a);
-                return hipGetLastError();
-            }
         // more rows than a lane's registers hold in four chunks: R rows a wave,
         // X from L2 (against the rows staged in LDS: fp16 W, M = 8, K = 2048,
         // N = 8192 15.4 -> 13.3 us; K = 3072, N = 768 9.8 -> 5.3; fp16 X,
-        // K = 1000, N = 3000 6.7 -> 4.2)
+        // K = 1000, N = 3000 6.7 -> 4.2), or staged after all
+        if constexpr (MP == 4 || sizeof(TW) == 4)
+            if (staged_x<MP, TI, TW>(a.K, a.N)) {
+                hipLaunchKernelGGL((slab_vec_kernel<MP, R, KCH, TI, TW>), dim3(blocks), dim3(256), 0, s, a);
+                return hipGetLastError();
+            }
         return launch_any<MP, TI, TW>(a, s);
     }
 }
