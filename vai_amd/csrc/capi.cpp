@@ -670,7 +670,9 @@ vai_status vai_conv2d_launch(const vai_conv2d_args* a, vai_stream_t stream)
         return hip_status(conv_launch(c, a->i_dtype, (hipStream_t)stream));
     }
     // rows and kernels the packed plan does not hold, over the weight as stored
-    if (a->w_dtype == VAI_DTYPE_F16 && conv_direct_ok(a->batch, a->ci, a->wi, a->co, ho, a->kernel, a->stride)) {
+    // (except where the gather below is faster)
+    if (a->w_dtype == VAI_DTYPE_F16 &&
+        conv_direct_ok(a->batch, a->ci, a->wi, a->co, ho, a->kernel, a->stride, a->i_dtype, plan_cus())) {
         ConvDirectParams c{};
         c.out = a->out; c.x = a->in; c.w = a->weight;
         c.bias = a->bias; c.scale = a->scale; c.residual = a->residual;

@@ -338,14 +338,48 @@ static uint32_t block_of(uint32_t ci, uint32_t ks, uint32_t stride, uint32_t ct,
 // 64 output channels and 4 rows a workgroup, or 32 and 8 (no idle waves) up to 32 channels.
 static uint32_t ct_of(uint32_t co) { return co <= 32 ? 32 : 64; }
 
+// Where the gather of gemm.hip takes less time than this kernel (us, gather /
+// this). A full chip is more workgroups than CUs can hold idle rows for free.
+static bool gather_faster(bool x32, uint32_t ci, uint32_t ho, uint32_t rows, uint32_t ctiles, uint64_t wgs, uint32_t ks,
+                          uint32_t stride, uint32_t cus)
+{
+    // Windows with gaps: the staging reads what no tap uses, once per 64 output
+    // channels. 1x1 stride 4, 256 -> 64, 40x132 22 / 65. 1x1 stride 2 pays off for
+    // one tile of channels (64 -> 64, 160x160 17.9 / 10.4) and where several leave
+    // CUs idle (64 -> 256, 40x132 13.2 / 10.6, 300x300 61 / 83; 512 -> 512, 8x136
+    // fp16 36.5 / 41, fp32 71 / 54), stride 3 with few fp16 channels (64 -> 64,
+    // 160x160 17.9 / 13.0, fp32 40x132 12.7 / 15.3); 3x3 stride 4 likewise (64 -> 64,
+    // 160x160 54 / 28; 64 -> 256, 85 / 98, 40x132 49 / 30).
+    if (stride > ks) {
+        if (ks == 1 && stride == 2) return ctiles > 1 && (x32 ? wgs > 2 * cus : ci >= 512 || wgs > cus);
+        if (ks == 1) return stride > 3 || x32 || ci > 64 || (ctiles > 1 && wgs > cus);
+        return ctiles > 1 && wgs > cus;
+    }
+    // Images of one row (of the 4 or 8 that a workgroup takes) that fill the chip:
+    // 3x3 stride 2, 512 -> 512, 8000 columns 352 / 562, stride 1 353 / 371 (4000
+    // columns 1 / 0.63; 64 -> 64, 64000, fp16 77 / 69); 5x5 stride 2, 64 -> 64, 64000
+    // columns 185 / 219. 1x1, whose gather is cheap, and strides as wide as the
+    // kernel, with up to a quarter of the rows (1x1 16 -> 32, 2x64000 23 / 27; 3x3
+    // stride 3, 4x64000 57 / 75); 1x1 with many channels beyond that (fp16 512 ->
+    // 512, 5x8000 174 / 212; fp32 2x8000 98 / 127, 3x8000 168 / 157).
+    const bool thin = 4 * (uint64_t)ho <= rows;
+    if (ks > 1 && stride == ks && thin && wgs > 2 * cus) return true;
+    if (wgs <= 4 * cus) return false;
+    if (ks == 1) return thin || (ci >= 256 && (x32 ? 2 * (uint64_t)ho <= rows : 8 * (uint64_t)ho <= 7 * (uint64_t)rows));
+    return ho == 1 && (ks == 3 ? stride > 1 || x32 || ci >= 256 : ks == 5 && stride > 1);
+}
+
 // Rows of at least one 8-column piece, weights of at least one 8-value piece,
 // and a grid of at most 65535 in y and z.
-bool conv_direct_ok(uint32_t batch, uint32_t ci, uint32_t wi, uint32_t co, uint32_t ho, uint32_t ks, uint32_t stride)
+bool conv_direct_ok(uint32_t batch, uint32_t ci, uint32_t wi, uint32_t co, uint32_t ho, uint32_t ks, uint32_t stride,
+                    int x_dt, uint32_t cus)
 {
-    const uint32_t ct = ct_of(co);
-    const uint64_t ytiles = (ho + cd::ph_of(ct) - 1) / cd::ph_of(ct), ctiles = (co + ct - 1) / ct;
+    const uint32_t ct = ct_of(co), ph = cd::ph_of(ct), wo = (wi - 1) / stride + 1;
+    const uint64_t ytiles = (ho + ph - 1) / ph, ctiles = (co + ct - 1) / ct;
     return wi >= 8 && ks <= 31 && stride <= 64 && (uint64_t)ci * ks * ks >= 8 && (uint64_t)ci * ks * ks < (1u << 24) &&
-           batch <= 65535 && ytiles * ctiles <= 65535 && block_of(ci, ks, stride, ct, 160 * 1024) > 0;
+           batch <= 65535 && ytiles * ctiles <= 65535 && block_of(ci, ks, stride, ct, 160 * 1024) > 0 &&
+           !gather_faster(x_dt == DT_F32, ci, ho, (uint32_t)ytiles * ph, (uint32_t)ctiles,
+                          batch * ytiles * ctiles * ((wo + cd::PW - 1) / cd::PW), ks, stride, cus);
 }
 
 template <typename TI, int CT, int KS>

@@ -285,7 +285,8 @@ struct ConvDirectParams {
     // set by the launch: channels per block, row tiles, multipliers for the kernel's divisions
     uint32_t cb, ytiles, m_kk, m_c8, m_nv, m_wv;
 };
-bool conv_direct_ok(uint32_t batch, uint32_t ci, uint32_t wi, uint32_t co, uint32_t ho, uint32_t ks, uint32_t stride);
+bool conv_direct_ok(uint32_t batch, uint32_t ci, uint32_t wi, uint32_t co, uint32_t ho, uint32_t ks, uint32_t stride,
+                    int x_dt, uint32_t cus);
 hipError_t conv_direct_launch(ConvDirectParams p, int x_dt, hipStream_t s);
 
 // Split-K fold for Linear: O = s*epi(sum_z P[z] + B) (+R).
