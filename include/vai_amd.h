@@ -87,8 +87,9 @@ typedef struct {
     uint32_t gated;
     uint32_t gate_epilogue;
     /* NULL, or vai_linear_pack_weight()'s output for this weight: fp16 I and W
-     * with M >= 3 then read W from that fragment-major copy (M of 512 and more
-     * straight into the matrix cores' registers). */
+     * with M >= 3 then read W from that fragment-major copy (256x256 tiles and 3-8
+     * rows straight into the matrix cores' registers, the small tiles through
+     * LDS; the other plans read W as stored). */
     const void* packed_weight;
     /* Accumulator dtype, Linear::setAccDtype (/root/reference/vai/nodes/
      * linear.h:289,2320): VAI_DTYPE_F32 (0, the default and the reference's
@@ -129,7 +130,7 @@ vai_status vai_linear_pack_weight(const vai_linear_args* args, void* packed, siz
                                   vai_stream_t stream);
 
 /* Which kernel vai_linear_launch picks for args (for tests and reports):
- * writes a short name ("slab", "slab_scalar", "tile_f16_128x128", ...). */
+ * writes a short name ("slab", "slab_any", "tile_f16_128x128", ...). */
 vai_status vai_linear_plan(const vai_linear_args* args, char* name, size_t name_len, uint32_t* split_count);
 
 /* GatedMul alone: O[r,j] = epi(I[r,j]) * I[r,H+j], I [rows, 2H].

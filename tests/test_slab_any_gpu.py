@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 F16, F32 = np.float16, np.float32
 
 
-def run(gpu, x, w, odt, xoff=0, woff=0, plan="slab_scalar"):
+def run(gpu, x, w, odt, xoff=0, woff=0, plan="slab_any"):
     D = gpu.DeviceArray.from_numpy
     dx = D(np.concatenate([np.full(xoff, np.nan, x.dtype), x.ravel(), np.full(9, np.nan, x.dtype)]))
     dw = D(np.concatenate([np.full(woff, np.nan, w.dtype), w.ravel(), np.full(9, np.nan, w.dtype)]))
@@ -43,7 +43,8 @@ def run(gpu, x, w, odt, xoff=0, woff=0, plan="slab_scalar"):
     (8, 512, 40, F32, F16, F32, (1, 0)),         # X off a boundary
     (6, 260, 21, F32, F32, F32, (3, 2)),
 ])
-def test_slab_any(gpu, m, k, n, xdt, wdt, odt, off, plan="slab_scalar"):
+def test_slab_any(gpu, m, k, n, xdt, wdt, odt, off, plan=None):
+    plan = plan or ("slab_any" if k >= 8 else "slab_scalar")
     rng = np.random.default_rng(m + k + n)
     x, w = draw((m, k), rng, xdt), draw(normal((n, k), 0.1), rng, wdt)
     got = run(gpu, x, w, odt, *off, plan=plan)

@@ -339,7 +339,7 @@ vai_status vai_linear_plan(const vai_linear_args* a, char* name, size_t name_len
         snprintf(buf, sizeof buf, "%s%s",
                  p.packed_gemv ? "slab_packed"
                  : (sp.M >= 5 && gemv_mfma_ok(sp)) ? "slab_mfma"
-                 : slab_vec_ok(sp) ? "slab" : "slab_scalar",
+                 : slab_vec_ok(sp) ? "slab" : slab_any_ok(sp) ? "slab_any" : "slab_scalar",
                  p.kind == LinearPlan::SlabThenGate ? "+gate" : "");
     } else if (p.kind == LinearPlan::Acc16Tile) {
         snprintf(buf, sizeof buf, "tile_acc16_64x64%s", a->gated ? "_gated" : "");

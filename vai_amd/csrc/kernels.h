@@ -21,6 +21,7 @@ struct SlabParams {
     float scalar_scale;
 };
 bool slab_vec_ok(const SlabParams& a);
+bool slab_any_ok(const SlabParams& a);
 bool gemv_mfma_ok(const SlabParams& a);
 hipError_t slab_launch(const SlabParams& a, hipStream_t s);
 // fp16 I and W, M <= 8, over the packed weight of gemm_pack_weight (same
@@ -136,9 +137,10 @@ size_t gemm_packed_weight_bytes(uint32_t N, uint32_t K, uint32_t H, bool gated);
 hipError_t gemm_pack_weight(void* dst, const void* w, uint32_t N, uint32_t K, uint32_t H, bool gated, hipStream_t s);
 hipError_t gemm_packed_launch(const GemmParams& p, const void* packed, bool gated, hipStream_t s);
 
-// The sizes between: any fp16 weight as stored, fp16 or fp32 X, small tiles
-// whose waves split K (gemm_ksplit.hip). gemm_ksplit_plan returns the tile for
-// a launch and its modelled time.
+// The sizes between, in small tiles whose waves split K (gemm_ksplit.hip): fp16
+// weights, as stored or packed, with fp16 or fp32 X, gated or not, and fp32 X and
+// W; K from 32 to 2^22, operands under 2^31 bytes and M N under 2^31.
+// gemm_ksplit_plan returns the tile for a launch and its modelled time.
 bool gemm_ksplit_ok(const GemmParams& p, bool gated);
 int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us);
 float gemm_ksplit_few_us(const GemmParams& p);   // the time of few small tiles

@@ -373,8 +373,9 @@ __global__ __launch_bounds__(256) void slab_any_kernel(SlabParams a)
     store_output(slab_output(a), (size_t)m * N + n0 + r, acc[0]);
 }
 
-// K shorter than one chunk, or elements off their own alignment: one wave per
-// output column, one element a lane.
+// K < 8 that slab_vec_ok does not take (slab_any_kernel's chunk of fp16 weights;
+// fp32 ones keep the same line), or elements off their own alignment: one wave
+// per output column, one element a lane.
 template <int MP>
 __global__ __launch_bounds__(256) void slab_scalar_kernel(SlabParams a)
 {
@@ -551,11 +552,20 @@ static hipError_t launch_m(const SlabParams& a, bool vec, hipStream_t s)
     return go(float{}, float{});
 }
 
+// Rows of whole 16-byte chunks (slab_reg_kernel, slab_vec_kernel, and with more
+// activations slab_any_kernel).
 bool slab_vec_ok(const SlabParams& a)
 {
     const uint32_t epc = a.w_dtype == DT_F16 ? 8 : 4;
     const size_t ib = a.i_dtype == DT_F16 ? 2 : 4;
     return a.K % epc == 0 && ((uintptr_t)a.weight % 16) == 0 && ((uintptr_t)a.in % (epc * ib)) == 0;
+}
+
+// Any other rows that slab_any_kernel takes.
+bool slab_any_ok(const SlabParams& a)
+{
+    const uintptr_t isz = a.i_dtype == DT_F16 ? 2 : 4, wsz = a.w_dtype == DT_F16 ? 2 : 4;
+    return a.K >= 8 && (uintptr_t)a.in % isz == 0 && (uintptr_t)a.weight % wsz == 0;
 }
 
 hipError_t slab_launch(const SlabParams& a, hipStream_t s)
@@ -569,9 +579,8 @@ hipError_t slab_launch(const SlabParams& a, hipStream_t s)
         hipLaunchKernelGGL(gemv_lds_kernel, dim3((a.N + 15) / 16), dim3(256), 65536, s, a);
         return hipGetLastError();
     }
-    const uintptr_t isz = a.i_dtype == DT_F16 ? 2 : 4, wsz = a.w_dtype == DT_F16 ? 2 : 4;
     const bool vec = slab_vec_ok(a);
-    if (vec || (a.K >= 8 && (uintptr_t)a.in % isz == 0 && (uintptr_t)a.weight % wsz == 0)) {
+    if (vec || slab_any_ok(a)) {
         switch (a.M) {
         case 1: return launch_m<1>(a, vec, s);
         case 2: return launch_m<2>(a, vec, s);
