@@ -81,3 +81,25 @@ def test_prefill_nan_key(gpu, hq, hkv, t, d):
     assert np.isnan(outs[1][0, j:, :g]).all()
     assert np.allclose(outs[1][0, :j], outs[0][0, :j], rtol=0, atol=2.0 ** -10 * np.abs(v.astype(F32)).max())
     assert (outs[1][0, :, g:] == outs[0][0, :, g:]).all()
+
+
+@pytest.mark.parametrize("d, count", [(64, 0), (128, 0), (128, 12), (128, 70), (64, 200)])
+def test_prefill_into_a_large_cache(gpu, d, count):
+    """A chunk over a cache that holds little of what it was made for: planned in long walks for two wave groups,
+    of which the second has nothing (one tile), or the last tile nothing for it."""
+    from oracle import oracle
+    rng = np.random.default_rng(d + count)
+    hq, hkv, t, size = 4, 2, 52, 8192
+    kc, vc = (draw((hkv, size, d), rng, F16) for _ in range(2))
+    kc[:, count:], vc[:, count:] = np.nan, np.nan          # rows never written
+    q, k, v = (draw((1, h, t, d), rng, F16) for h in (hq, hkv, hkv))
+    D = gpu.DeviceArray.from_numpy
+    out = gpu.DeviceArray((1, t, hq, d), F32)
+    out.fill_(0xFF)
+    print(f"prefill chunk d={d} count={count}", flush=True)
+    got = gpu.attention(out, D(q), D(k), D(v), causal=True,
+                        cache=(D(kc), D(vc), D(np.array([count], np.uint32)), False)).numpy()
+    want, _, _ = oracle.attention_cached(q[0], k, v, kc, vc, count, causal=True)
+    # P to fp16 (2^-11 of sum p |v| <= max |v|), scores of D products in fp32
+    vmax = max(np.abs(vc[:, :count]).max(initial=0), np.abs(v).max())
+    assert np.isfinite(got).all() and np.abs(got[0] - want).max() <= float(vmax) * (2.0 ** -11 + 64 * d * 2.0 ** -24)

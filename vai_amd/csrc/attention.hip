@@ -571,7 +571,9 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 
         LDS_AS float4v* po = (LDS_AS float4v*)(all + L::BYTES + wave * (QW * D * 4)) + lane;
         typedef float float2v __attribute__((ext_vector_type(2)));
         LDS_AS float2v* pm = (LDS_AS float2v*)(all + wave * (QW * D * 4)) + lane;   // within wave's own rows below
-        if (kg == 1) {
+        // (after a walk of one tile, as over an empty cache, it has nothing to hand over)
+        const bool both = ntiles > 1;
+        if (both && kg == 1) {
             *pm = float2v{m, l};
 #pragma unroll
             for (int d = 0; d < DF; ++d)
@@ -579,21 +581,23 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 
                 for (int q4 = 0; q4 < 4; ++q4)
                     po[(d * 4 + q4) * 64] = float4v{o[d][4 * q4], o[d][4 * q4 + 1], o[d][4 * q4 + 2], o[d][4 * q4 + 3]};
         }
-        __syncthreads();
+        if (both) __syncthreads();
         if (kg == 1) return;
-        const float2v ml = *pm;
-        const float mm = fmaxf(m, ml[0]), mr = mm == -__builtin_inff() ? 0.f : mm;
-        const float a0 = __builtin_amdgcn_exp2f(m - mr), a1 = __builtin_amdgcn_exp2f(ml[0] - mr);
-        l = l * a0 + ml[1] * a1;
-        m = mm;
+        if (both) {
+            const float2v ml = *pm;
+            const float mm = fmaxf(m, ml[0]), mr = mm == -__builtin_inff() ? 0.f : mm;
+            const float a0 = __builtin_amdgcn_exp2f(m - mr), a1 = __builtin_amdgcn_exp2f(ml[0] - mr);
+            l = l * a0 + ml[1] * a1;
+            m = mm;
 #pragma unroll
-        for (int d = 0; d < DF; ++d)
+            for (int d = 0; d < DF; ++d)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const float4v v = po[(d * 4 + q4) * 64];
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const float4v v = po[(d * 4 + q4) * 64];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[d][4 * q4 + e] = o[d][4 * q4 + e] * a0 + v[e] * a1;
-            }
+                    for (int e = 0; e < 4; ++e) o[d][4 * q4 + e] = o[d][4 * q4 + e] * a0 + v[e] * a1;
+                }
+        }
     }
 
     // Output: a partial when the key range is split, else O / l. A partial
