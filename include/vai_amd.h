@@ -236,8 +236,8 @@ vai_status vai_attn_scores_launch(const vai_attn_scores_args* args, vai_stream_t
  *   flash-attention gate, attention.h:916-945) and 16-byte aligned operands
  *   take the MFMA flash kernel: fp32 softmax statistics and accumulation,
  *   Q.K^T and P.V on fp16 operands (fp32 Q is rounded to fp16 as the
- *   reference's f16-staged tiles do, fp32 K / V are rounded too, into workspace
- *   copies first where there are many query rows, P enters P.V as fp16). Every other head dim takes a plain
+ *   reference's f16-staged tiles do, fp32 K / V are rounded into workspace
+ *   copies first, P enters P.V as fp16). Every other head dim takes a plain
  *   fp32 kernel (the reference's naive attention.comp role).
  *   Long key ranges may be split over workgroups and merged; fp32 K / V and
  *   the split need vai_attention_workspace_size() bytes of workspace.
@@ -283,10 +283,9 @@ typedef struct {
 
 vai_status vai_attention_launch(const vai_attention_args* args, vai_stream_t stream);
 /* Bytes of workspace a launch needs: nonzero when fp32 K / V take the flash
- * kernel (their fp16 copies; a few query rows per KV head read them as they
- * are), or when the query tiles alone do not fill the GPU and long key ranges
- * are split over workgroups (partial results merged by a second pass, the
- * split-K of attention-fa-reduce.comp). */
+ * kernel (their fp16 copies), or when the query tiles alone do not fill the
+ * GPU and long key ranges are split over workgroups (partial results merged by
+ * a second pass, the split-K of attention-fa-reduce.comp). */
 size_t vai_attention_workspace_size(const vai_attention_args* args);
 
 /* ---------------------------------------------------------------------------

@@ -124,32 +124,3 @@ def test_decode_graph_follows_the_count(gpu):
         want, wkc, _ = oracle.attention_cached(q[0], k, v, kc, vc, count, causal=True)
         assert_close(out.numpy()[0], want, FP16)
         np.testing.assert_array_equal(dkc.numpy(), wkc)
-
-
-@pytest.mark.parametrize("d, hq, hkv, tq, size, cdt", [(128, 8, 2, 1, 4096, F32), (64, 8, 8, 2, 2048, F16),
-                                                       (256, 4, 1, 3, 2048, F32)])
-def test_decode_workspace(gpu, d, hq, hkv, tq, size, cdt):
-    """The workspace asked for is what the launch uses: the units' partial sums, no fp16 copy of an fp32 cache; the
-    bytes after it stay as they were, and less is refused."""
-    rng = np.random.default_rng(d)
-    count = size - 100
-    kc, vc = _cache_planes(rng, hkv, size, d, count, False, cdt)
-    q, k, v = draw((1, hq, tq, d), rng, F16), draw((1, hkv, tq, d), rng, F16), draw((1, hkv, tq, d), rng, F16)
-    D = gpu.DeviceArray.from_numpy
-    dkc, dvc, dq, dk, dv, cnt = D(kc), D(vc), D(q), D(k), D(v), D(np.array([count], np.uint32))
-    out = gpu.DeviceArray((1, tq, hq, d), F32)
-    a = gpu.attention_args(out, dq, dk, dv, causal=True, cache=(dkc, dvc, cnt, False))
-    need = gpu.lib().vai_attention_workspace_size(ctypes.byref(a))
-    unit = hkv * (hq // hkv * tq) * ((64 if d <= 64 else 128 if d <= 128 else 256) + 2) * 4
-    print(f"decode workspace d={d} size={size} {np.dtype(cdt)}: {need} = {need / unit} units", flush=True)
-    assert 1 < need // unit <= 256 and need % unit == 0
-    ws = gpu.DeviceArray((need + 4096,), np.uint8)
-    ws.fill_(0xA5)
-    a.workspace, a.workspace_bytes = ws.ptr, need - 4
-    assert gpu.lib().vai_attention_launch(ctypes.byref(a), None) == 1004
-    a.workspace_bytes = need
-    gpu.check(gpu.lib().vai_attention_launch(ctypes.byref(a), None), "attention")
-    gpu.synchronize()
-    assert (ws.numpy()[need:] == 0xA5).all()
-    want, _, _ = oracle.attention_cached(q[0], k, v, kc, vc, count, causal=True)
-    assert_close(out.numpy()[0], want, FP16)

@@ -1006,12 +1006,8 @@ void attention_plan(AttnParams& p, uint32_t cus)
     p.key_groups = flash_key_groups(p, cus);
 }
 
-// (the decode kernel's plan keeps within what the flash plan would ask for, and
-// reads fp32 K and V as they are)
-size_t attention_workspace_bytes(const AttnParams& p)
-{
-    return p.dec_units ? attention_decode_workspace(p, p.dec_units) : flash_workspace(p);
-}
+// (the decode kernel's plan keeps within what the flash plan asks for)
+size_t attention_workspace_bytes(const AttnParams& p) { return flash_workspace(p); }
 
 void attention_set_workspace(AttnParams& p, void* ws)
 {
