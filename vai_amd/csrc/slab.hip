@@ -488,21 +488,23 @@ static hipError_t launch_any(const SlabParams& a, hipStream_t s)
 // Which of the calls with more activations than a lane holds ahead stage X in
 // LDS (slab_vec_kernel) and which read it from L2 (slab_any_kernel). Measured,
 // us, staged / from L2. Long and many rows, where a wave reads twice the bytes
-// of its W as X: X fp32, W fp16, 4 rows, K = 4096, N = 16384 29.6 / 36.9, K = 8192,
-// N = 32768 99 / 186, but K = 6400, N = 6144 21.8 / 20.2, K = 2048, N = 4096 8.3 /
-// 7.6; W fp32, 4 rows, K = 6400, N = 16384 65 / 86, 8 rows, K = 2048, N = 4096 11.3 /
+// of its W as X: X fp32, W fp16, 4 rows, K = 4096, N = 16384 29.6 / 36.9, K = 8120,
+// N = 6144 1 / 1.52 (erratic: K = 6400 1 / 0.93), but K = 2048, N = 4096 8.3 / 7.6;
+// W fp32, 4 rows, K = 6400, N = 16384 65 / 86, 8 rows, K = 2048, N = 4096 11.3 /
 // 11.6-12.7, but N = 1024 8.1 / 7.3. fp32 rows of one K block (512 to 1024
 // elements), which are read from L2 in three or four passes: 5 rows, K = 1000, N =
 // 2048 4.5 / 5.5, 4 rows, N = 8192 7.3 / 8.6, but 5 rows, K = 768, N = 8192 8.7 / 7.8.
+// Few workgroups of four rows each: 5 rows, fp16 W, N = 2048, K = 2048, 4096 and
+// 8192 1 / 1.12, 1.00 and 1.08.
 template <int MP, typename TI, typename TW>
 static bool staged_x(uint32_t K, uint32_t N)
 {
     constexpr bool x32 = sizeof(TI) == 4, w32 = sizeof(TW) == 4;
     if (MP == 4) {
-        if (!w32) return K >= 3500 && N >= (K < 4608 ? 3072u : K < 8192 ? 16384u : 6144u);
+        if (!w32) return K > 3072 && N >= 3072;
         return (K > 768 && K < 1024) || (K >= 2048 && N >= 12288);
     }
-    if (!w32) return false;
+    if (!w32) return x32 && N >= 2048 && N < 3072 && K >= 2048 && (K < 2560 || K >= 5120);
     if (N >= 2048 && K > 512) return K >= 1024 || N < (x32 ? 8192u : 3072u);
     return x32 && K >= 1024 && N >= 1536 && (uint64_t)N * K >= 5500000;
 }
@@ -529,7 +531,7 @@ static hipError_t launch_vec(const SlabParams& a, hipStream_t s)
         // X from L2 (against the rows staged in LDS: fp16 W, M = 8, K = 2048,
         // N = 8192 15.4 -> 13.3 us; K = 3072, N = 768 9.8 -> 5.3; fp16 X,
         // K = 1000, N = 3000 6.7 -> 4.2), or staged after all
-        if constexpr (MP == 4 || sizeof(TW) == 4)
+        if constexpr (sizeof(TI) == 4 || sizeof(TW) == 4)
             if (staged_x<MP, TI, TW>(a.K, a.N)) {
                 hipLaunchKernelGGL((slab_vec_kernel<MP, R, KCH, TI, TW>), dim3(blocks), dim3(256), 0, s, a);
                 return hipGetLastError();
