@@ -115,12 +115,13 @@ namespace {
 // The packed 256x256 kernel's time (us) on g: rounds of units, 1.77 us per
 // 64-wide k stage (config 3: 512 tiles, 48 stages, 177 us), and with a K split
 // the reduce launch and its passes over the partial planes (M = 2000,
-// K = N = 2048 in 4 splits: 43 us, of which the planes are 20).
+// K = N = 2048 in 4 splits: 43 us, of which the planes are 20); split launches
+// take nine tenths of that ([400, 8192], N 8192 75 us, [339, 3072], N 15360 62).
 float packed_us(const GemmParams& g, bool gated, uint32_t tiles)
 {
     const uint32_t S = gated ? 1 : g.splits, rounds = (tiles * S + plan_cus() - 1) / plan_cus();
     const float us = 2.5f + rounds * (4.f + 1.77f * (float)(g.K / S) / 64.f);
-    return S == 1 ? us : us + 4.f + (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 4e6f;
+    return S == 1 ? us : .9f * (us + 4.f + (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 4e6f);
 }
 
 // The generic tiles, with a K split where even the smallest leave CUs idle.
@@ -181,12 +182,12 @@ LinearPlan plan_tile(const vai_linear_args* a)
 // 23.4; K 7864 25.9 / 37.2.
 float split_us(const GemmParams& g, uint32_t S)
 {
-    const float planes = (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 2e6f;
+    const float planes = (float)(S + 1) * 4.f * (float)g.M * (float)g.N / 1e6f;
     const bool aligned = (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
     if (g.b_dtype == VAI_DTYPE_F32)
-        return 2.f + .265f * (float)S + (g.K % 4 == 0 && aligned ? .062f : .08f) * (float)(g.K / S) + planes;
+        return 2.f + .265f * (float)S + (g.K % 4 == 0 && aligned ? .062f : .07f) * (float)(g.K / S) + planes / 1.5f;
     return 3.f + (aligned ? .3f : .27f) * (float)S +
-           (g.K % 8 != 0 ? .11f : aligned ? .028f : .05f) * (float)(g.K / S) + planes;
+           (g.K % 8 != 0 ? .11f : aligned ? .028f : .05f) * (float)(g.K / S) + planes / 2.f;
 }
 
 LinearPlan plan_linear(const vai_linear_args* a)
@@ -259,14 +260,18 @@ LinearPlan plan_linear(const vai_linear_args* a)
         }
         // fp32 problems with fewer 64x64 tiles than CUs, or where its rounds of
         // 32-row tiles still take less: one launch over the full K with a
-        // CU-filling tile count. Over more than 16 rounds of 16 columns the
-        // operands' repeated reads count: 17 to 25 rounds of K = 4736 to 7424 took
-        // 1.1-1.8 times the model ([524, 6656], N 5832 714 us; in 32x32 tiles,
-        // whose sums are as exact, 411).
+        // CU-filling tile count. Over more than 11 rounds of 16 columns the
+        // operands' repeated reads count: 13 to 25 rounds took 1.1-1.8 times the
+        // model ([524, 6656], N 5832 714 us, [2123, 4416], N 768 245; in 32x32
+        // tiles, whose sums are as exact, 411 and 165).
         const int nf = gemm_f32_nf(M, N, plan_cus());
         const uint32_t rounds = (tiles_of(M, N, 32, 16 * nf) + plan_cus() - 1) / plan_cus();
         float f32_us = 2.5f + (float)rounds * (2.f + 0.0022f * (float)nf * (float)K);
-        if (nf == 1 && rounds > 16 && p.ks_tile == 0) f32_us *= 1.3f;
+        if (ksplit && nf == 1 && rounds > 11 && a->w_dtype == VAI_DTYPE_F32 &&
+            gemm_ksplit_tile_us(g, false, plan_cus(), 0) < 1.3f * f32_us) {
+            p.ks_tile = 0;
+            f32_us = 1e30f;
+        }
         if (a->split_size == 0 && !a->gated && gemm_f32_ok(g) &&
             (tiles_of(M, N, 64, 64) < plan_cus() || !ksplit || f32_us <= ksplit_us)) {
             p.kind = LinearPlan::F32Small;

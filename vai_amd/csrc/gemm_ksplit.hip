@@ -627,20 +627,25 @@ void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn)
     bn = ks::TILES[tile].bn;
 }
 
-int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
+float gemm_ksplit_tile_us(const GemmParams& p, bool gated, uint32_t cus, int tile)
 {
     const int x = p.b_dtype == DT_F32 ? 2 : p.a_dtype == DT_F16 ? 0 : 1;
     // (register staging: fp16 1.5-1.9; fp32 measured alike, 15.2 us a tile at K = 767 and 768)
     const float chunks = (float)((p.K + 63) / 64) * (ks::dma_ok(p) || x == 2 ? 1.f : 1.7f);
     const uint32_t cols = gated ? 2 * p.H : p.N;
+    const ks::Tile& k = ks::TILES[tile];
+    const uint64_t tiles = (uint64_t)((p.M + k.bm - 1) / k.bm) * ((cols + k.bn - 1) / k.bn);
+    // (fp32 quadrants alone on a CU, one wave per SIMD: 22 us where a pair takes 2 x 19)
+    const float rounds = (float)((tiles + cus - 1) / cus) * (x == 2 && k.bm == 64 && tiles <= cus ? 1.15f : 1.f);
+    return 2.5f + rounds * (k.fixed[x] + chunks * k.chunk[x]);
+}
+
+int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us)
+{
     int best = 0;
     *us = 1e30f;
     for (int t = 0; t < ks::NTILES; ++t) {
-        const ks::Tile& k = ks::TILES[t];
-        const uint64_t tiles = (uint64_t)((p.M + k.bm - 1) / k.bm) * ((cols + k.bn - 1) / k.bn);
-        // (fp32 quadrants alone on a CU, one wave per SIMD: 22 us where a pair takes 2 x 19)
-        const float rounds = (float)((tiles + cus - 1) / cus) * (x == 2 && k.bm == 64 && tiles <= cus ? 1.15f : 1.f);
-        const float cost = 2.5f + rounds * (k.fixed[x] + chunks * k.chunk[x]);
+        const float cost = gemm_ksplit_tile_us(p, gated, cus, t);
         if (cost < *us) { *us = cost; best = t; }
     }
     return best;

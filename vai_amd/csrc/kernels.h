@@ -143,6 +143,7 @@ hipError_t gemm_packed_launch(const GemmParams& p, const void* packed, bool gate
 // gemm_ksplit_plan returns the tile for a launch and its modelled time.
 bool gemm_ksplit_ok(const GemmParams& p, bool gated);
 int gemm_ksplit_plan(const GemmParams& p, bool gated, uint32_t cus, float* us);
+float gemm_ksplit_tile_us(const GemmParams& p, bool gated, uint32_t cus, int tile);
 float gemm_ksplit_few_us(const GemmParams& p);   // the time of few small tiles
 void gemm_ksplit_tile(int tile, uint32_t& bm, uint32_t& bn);   // bn: logical columns (gated: gate and up)
 // packed: null, or gemm_pack_weight's copy of an fp16 weight for fp16 X
