@@ -230,7 +230,11 @@ LinearPlan plan_linear(const vai_linear_args* a)
         // whatever the 256x256 kernels do not take, and where it is faster
         // than the packed one below 512 rows or when that would need more than
         // 8 K splits (their planes then cost more than the product: M = 608,
-        // K = 3072, N = 896 in 12 splits 124 us against 19).
+        // K = 3072, N = 896 in 12 splits 125 us against 14). The line at 512
+        // rows is where the comparison was made, not where the times cross
+        // (packed / small tiles, us: 511 and 512 x 2048 x 2048 23 / 10.5, 2048 x
+        // 2048 x 2048 42 / 28, 1500 x 4096 x 4096 68 / 77, 2000 x 3072 x 5120,
+        // unsplit, 71 / 86 in the 256x256 tiles over the weight as stored).
         float ksplit_us = 0.f;
         const bool ksplit = a->split_size == 0 && gemm_ksplit_ok(g, a->gated != 0);
         if (ksplit) p.ks_tile = gemm_ksplit_plan(g, a->gated != 0, plan_cus(), &ksplit_us);

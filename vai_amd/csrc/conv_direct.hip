@@ -18,12 +18,14 @@
 // read hit distinct banks. The weights' taps are spread from their stored
 // order, c k k + tap, by two-byte LDS writes, once per workgroup and block.
 //
-// What is left after that is the address and transpose work of staging (about
-// half of a workgroup's time at 3x3: divisions are multiplications by
-// constants of the launch, the loads share one offset where rows are whole
-// aligned pieces) and one exposed memory latency per block. Measured against
-// the generic gather kernel (conv as a GEMM of gemm.hip, us): 32 -> 64
-// channels, stride 2, 320x320 33.7 -> 10.2; 64 -> 64, 160x160 55.7 -> 13.0;
+// What is left after that is latency: at 32 -> 64 channels, stride 2, 320x320
+// (200 workgroups, one a CU, all channels in one block) load, transpose, barrier
+// and MFMAs follow each other; a wave waits for its loads and at the barriers
+// 53% of the time and for an issue slot 22%, the VALU (addresses and transpose:
+// divisions are multiplications by constants of the launch, the loads share one
+// offset where rows are whole aligned pieces) works 13%, LDS 3% and the matrix
+// cores 3%. Measured against the generic gather kernel (conv as a GEMM of
+// gemm.hip, us): that 33.7 -> 9.7; 64 -> 64, 160x160 55.7 -> 13.0;
 // 1x1 17.5 -> 7.6; 16 -> 16, 320x320, fp32 image 52.7 -> 12.6; 32 -> 32,
 // 333x333 72 -> 18.6. Reading the window untransposed, 8 two-byte LDS reads a
 // lane and fragment, took 21 for the first.

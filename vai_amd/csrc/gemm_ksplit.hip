@@ -2,9 +2,13 @@
 // the 256x256 tiles: X (fp16 or fp32) . W^T (fp16, as stored), any N and K,
 // fused gate/up included.
 //
-// What bounds these sizes is bytes into the CUs (W and X each pass through
-// LDS once per workgroup, about 45 bytes a cycle and CU) and how many CUs have
-// work, not MFMA rate. So the output is cut into small tiles (32x32 to
+// What bounds these sizes is bytes into the CUs (W and X each pass through LDS
+// once per workgroup) and how many CUs have work, not MFMA rate: a full grid of
+// 32x32 tiles moves 50 bytes a cycle and CU (8.7 us per MB of a workgroup's
+// operands); where a CU has one workgroup of four waves (M = 61: 160 tiles of
+// 32x64; X fp32, M = 500: 256 of 64x64) it moves 21-24, its waves issuing 40% of
+// the time, waiting for their copies 36-40% and for an issue slot 20-23%, the
+// matrix cores 13% busy. So the output is cut into small tiles (32x32 to
 // 128x128, chosen by gemm_ksplit_plan so that the tiles fill the CUs), and the
 // 4 or 8 waves of a workgroup split K instead of the tile: every wave runs the
 // whole tile over its own 64- or 32-wide k chunks, dealt out in turn, so each
@@ -24,17 +28,16 @@
 //
 // Measured (back-to-back calls, us, against the kernels these sizes took
 // before, register-staged 64x64 tiles or 256x256 packed tiles with a K split):
-// X fp16 [61, 3072], N 5120 20.2 -> 11.1 (2.9 TB/s of W); fp32 [500, 2048],
-// N 2048 65.2 -> 15.0; fp16 [300, 4096], N 1000 146 -> 12; fp16 [948, 2481],
-// N 1216 (odd K) 205 -> 28; gated fp16 [500, 2048], H 2048 71 -> 16. At 32x32
-// a workgroup moves 8.7 us per MB of its operands, 50 bytes a cycle.
+// X fp16 [61, 3072], N 5120 21.5 -> 10.7 (2.9 TB/s of W); fp32 [500, 2048],
+// N 2048 62 -> 15.8; fp16 [300, 4096], N 1000 139 -> 11.4; fp16 [948, 2481],
+// N 1216 (odd K) 206 -> 31; gated fp16 [500, 2048], H 2048 54 -> 17.3.
 //
 // fp32 X and W (F32): v_mfma_f32_32x32x2_f32, a sixteenth of the rate, so the
 // matrix cores bound it and 64x64 quadrants are large enough (two workgroups a
-// CU; four sums per output). Against the register-staged 16x16x4 tiles with a
-// K split that these sizes took: [512, 768], N 3072 47.6 -> 32.6 us, 1024 rows
-// 78 -> 51 (94 of the 153 TFLOP/s a large product reaches); [600, 2048], N 2048
-// 107 -> 54; [900, 767], N 3073 124 -> 48; [100, 1147], N 3000 31 -> 16.
+// CU; four sums per output). Against the register-staged tiles that these sizes
+// took: [1024, 768], N 3072 75.5 -> 48.9 us; [1000, 3072], N 4096 579 -> 216 (117
+// of the 153 TFLOP/s that a large product reaches); [900, 767], N 3073 123 -> 49.7; [100, 1147], N
+// 3000 31.6 -> 16.3.
 //
 // Rows that are not whole 16-byte chunks (K % 8 != 0, fp32 K % 4) or operands off a
 // 16-byte boundary take the same kernel with the chunks loaded into registers
