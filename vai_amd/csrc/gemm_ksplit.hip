@@ -36,8 +36,8 @@
 // matrix cores bound it and 64x64 quadrants are large enough (two workgroups a
 // CU; four sums per output). Against the register-staged tiles that these sizes
 // took: [1024, 768], N 3072 75.5 -> 48.9 us; [1000, 3072], N 4096 579 -> 216 (117
-// of the 153 TFLOP/s that a large product reaches); [900, 767], N 3073 123 -> 49.7; [100, 1147], N
-// 3000 31.6 -> 16.3.
+// of the 153 TFLOP/s that a large product reaches); [900, 767], N 3073 123 -> 49.7;
+// [100, 1147], N 3000 31.6 -> 16.3.
 //
 // Rows that are not whole 16-byte chunks (K % 8 != 0, fp32 K % 4) or operands off a
 // 16-byte boundary take the same kernel with the chunks loaded into registers

@@ -7,8 +7,8 @@
 // Design (gfx950): W dominates the traffic (N*K elements, read once), so the
 // kernel is shaped for HBM: each wave owns R whole rows of W and issues all
 // of its 16-byte non-temporal loads for a K block before touching them, so a
-// CU keeps ~100 KB of loads in flight. The M <= 8 input rows are staged once
-// per workgroup in LDS and broadcast to the four waves. Each lane ends with
+// CU keeps ~100 KB of loads in flight. The M <= 8 input rows come from L2 (or
+// are staged once per workgroup in LDS where that is cheaper). Each lane ends with
 // M*R partial dot products; a butterfly over the wave halves the number of
 // values per lane at each exchange (M*R + 6 - log2(M*R) shuffles instead of
 // 6*M*R), leaving lane groups that each own one output for the epilogue.
