@@ -292,3 +292,25 @@ def test_attention_kv_cache_rejects(gpu):
     out2 = D((2, 2, 4, 64), np.float32)
     a = gpu.attention_args(out2, q2, k2, k2, cache=(kc, kc, cnt, False))  # one counter: batch 1 only
     assert gpu.lib().vai_attention_launch(ctypes.byref(a), None) == 1002
+
+
+@pytest.mark.parametrize("d, hq, hkv, tq, size, count, ring, span", [
+    (64, 8, 2, 130, 3132, 2718, False, 371),      # windows that start elsewhere in a key tile than those of a
+    (64, 8, 2, 130, 1377, 848, False, 83),        # full cache, which the split's chunks are counted for
+    (128, 16, 8, 33, 256, 319, True, 224),
+    (256, 4, 2, 33, 256, 506, True, 224),
+    (72, 4, 2, 340, 2304, 2836, True, 225),
+    (128, 4, 2, 130, 2048, 1000, False, 0),
+])
+def test_cached_window_at_any_count(gpu, d, hq, hkv, tq, size, count, ring, span):
+    """A chunk of queries over a cache sees every key of its window, however the count lies to the key tiles."""
+    rng = np.random.default_rng(d + count)
+    kc, vc = _cache_planes(rng, hkv, size, d, count, ring, np.float16)
+    q, k, v = (draw((1, h, tq, d), rng, np.float16) for h in (hq, hkv, hkv))
+    D = gpu.DeviceArray.from_numpy
+    out = gpu.DeviceArray((1, tq, hq, d), np.float32)
+    print(f"cached window d={d} tq={tq} size={size} count={count} ring={ring} span={span}", flush=True)
+    got = gpu.attention(out, D(q), D(k), D(v), causal=True, span=span,
+                        cache=(D(kc), D(vc), D(np.array([count], np.uint32)), ring)).numpy()
+    want, _, _ = oracle.attention_cached(q[0], k, v, kc, vc, count, ring=ring, causal=True, span=span)
+    assert_close(got[0], want, FP16)

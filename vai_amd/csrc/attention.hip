@@ -271,12 +271,13 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 
     // the branch that first uses it)
     asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.tq), "s"(p.tkv), "s"(p.head_dim), "s"(p.hq),
                  "s"(p.hkv), "s"(p.units), "s"(p.q_dtype), "s"(p.chunk_tiles));
-    uint32_t unit, h, b, qt, chunk = 0;
+    uint32_t unit, h, b, qt, chunk = 0, chunks = 1;
     if (p.units != 0) {
         // the plan's table: one entry per workgroup of the 1-D grid
         const uint32_t e0 = p.wg_tab[2 * blockIdx.x], e1 = p.wg_tab[2 * blockIdx.x + 1];
         qt = e0 & 0xFFFF;
         chunk = (e0 >> 16) & 0xFF;
+        chunks = e0 >> 24;
         unit = e1 & 0x3FF;
         h = (e1 >> 10) & 0x3FF;
         b = e1 >> 20;
@@ -297,6 +298,7 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 
     }
     qt = __builtin_amdgcn_readfirstlane(qt);
     chunk = __builtin_amdgcn_readfirstlane(chunk);
+    chunks = __builtin_amdgcn_readfirstlane(chunks);
     const uint32_t q0 = qt * BQ;
     const uint32_t hk = h / (p.hq / p.hkv);
     const uint32_t qsz = p.q_dtype == DT_F32 ? 4 : 2;
@@ -337,12 +339,14 @@ __global__ __launch_bounds__(256 * KG, KG == 2 ? 2 : D == 64 ? 3 : D == 128 ? 2 
         }
     }
 
-    // visible key tiles of the query tile, then this unit's chunk of them
+    // Visible key tiles of the query tile, then this unit's chunk of them. The
+    // last chunk goes to the end: the plan counted the tiles for a full cache,
+    // and a window that starts elsewhere in a tile can touch one more.
     int64_t tb, te;
     fa_tile_range(p, qt, cached, tb, te);
     if (p.units != 0) {
         const int64_t c0 = tb + (int64_t)chunk * p.chunk_tiles;
-        te = std::min<int64_t>(te, c0 + p.chunk_tiles);
+        if (chunk + 1 < chunks) te = std::min<int64_t>(te, c0 + p.chunk_tiles);
         tb = c0;
     }
     const int ntiles = (int)__builtin_amdgcn_readfirstlane((int)std::max<int64_t>(te - tb, 0));
